@@ -65,6 +65,24 @@ def test_random_targets():
     _check(got, ref)
 
 
+@pytest.mark.parametrize("n_fast,n_targets", [(1, 65), (255, 64), (256, 63), (257, 1), (1025, 130)])
+def test_sample_and_target_remainders(n_fast, n_targets):
+    # A wave takes 256 samples of a line and 64 targets at a time.  Worst case
+    # per unit of sigma: 1.25e-7 of the hardware sine, 1e-7 of the FP32 phase,
+    # one rounding per summed target.
+    rng = np.random.default_rng(n_fast + n_targets)
+    p = native.SarParams.reference_defaults()
+    p.La, p.H, p.Ntarget = 70.0, 3000.0, n_targets
+    pt = np.stack([rng.uniform(-60, 60, n_targets), rng.uniform(7000, 7000 + n_fast, n_targets),
+                   rng.uniform(0.2, 2.0, n_targets)], 1).astype(np.float32)
+    ta = np.linspace(-0.3, 0.3, 37).astype(np.float32)
+    t0 = np.float32(2 * math.sqrt(7000.0 ** 2 + p.H ** 2) / p.c)
+    tr = (t0 + np.arange(1, n_fast + 1, dtype=np.float32) / np.float32(p.Fr)).astype(np.float32)
+    got = _gen(pt, ta, tr, p)
+    ref = E.generate_echo(pt, ta, tr, p)
+    assert np.max(np.abs(got - ref)) <= 4e-7 * pt[:, 2].sum()
+
+
 def test_rejects_bad_arguments():
     import torch
     lib = native.load()
