@@ -235,12 +235,14 @@ const char* sarbp_last_error_detail(void);
 /* Kernel configuration knobs chosen by the autotuner.  A workgroup's tile is
  * (64 cols_per_lane) x (4 rows_per_lane) pixels: each lane accumulates
  * cols_per_lane columns (64 apart) of rows_per_lane rows.  pulses_per_stage
- * is the number of pulses staged in LDS per barrier interval, an upper bound:
- * the planner reduces it until the stage fits 64 KiB of LDS, then by one
- * pulse at a time while one pulse fewer lets one more workgroup share a CU
- * (a job's window sets the LDS per pulse), down to 4 pulses for a plain
- * launch (sarbp_plan_get_info reports the depth planned) and to 1 for a job
- * of a batch or a server, whose persistent launch gains more from occupancy.
+ * is the number of pulses whose planned windows the LDS of a barrier interval
+ * is sized for, an upper bound: the planner reduces it until the stage fits
+ * 64 KiB of LDS, then by one pulse at a time while one pulse fewer lets one
+ * more workgroup share a CU (a job's window sets the LDS per pulse), down to
+ * 4 pulses for a plain launch (sarbp_plan_get_info reports the depth planned)
+ * and to 1 for a job of a batch or a server.  Linear and sinc8 launches of
+ * SARBP_PREC_REF take at most the LDS that lets 4 workgroups share a CU, and
+ * pack it with as many pulses as fit at the length they touch.
  * The depth changes no bit of an image.  Shapes: rows 2, 4 or 8 with
  * cols 1 or 2; rows 2 or 4 with cols 4 (SARBP_PREC_REF); cols 1 otherwise. */
 typedef struct sarbp_tuning {
@@ -290,7 +292,9 @@ sarbp_status sarbp_get_tuning(sarbp_context* ctx, int32_t interp,
  * the grid alone -- a disc of the tile's radius, other classes and other
  * best tunings -- and keep their own per-class entries: the built-in
  * position-free defaults, or what sarbp_autotune without h_pos stored; an
- * all-class sarbp_set_tuning applies to both. */
+ * all-class sarbp_set_tuning applies to both.  A call that takes a built-in
+ * default of one column and 4 rows per lane for linear or sinc8 REF imaging
+ * runs 8 rows on an image of 5120 or more 64 x 32 tiles. */
 sarbp_status sarbp_set_class_tuning(sarbp_context* ctx, int32_t interp,
                                     int32_t precision, int32_t dtype,
                                     int32_t size_class, const sarbp_tuning* tuning);

@@ -90,13 +90,15 @@ struct sarbp_plan {
 namespace sarbp {
 
 // The context's tuning of a class, else its all-classes tuning, else the
-// built-in default (`positions`: for a plan that knows the antenna positions).
-sarbp_tuning get_tuning(sarbp_context* ctx, int interp, int prec, int dtype, int cls, bool positions = true) {
+// built-in default (`positions`: for a plan that knows the antenna positions;
+// `g`: the job's grid, NULL for the class alone).
+sarbp_tuning get_tuning(sarbp_context* ctx, int interp, int prec, int dtype, int cls, bool positions = true,
+                        const sarbp_grid* g = nullptr) {
   auto it = ctx->tuning.find(tuning_key(interp, prec, dtype, cls, positions));
   if (it != ctx->tuning.end()) return it->second;
   it = ctx->tuning.find(tuning_key(interp, prec, dtype, kAllClasses));
   if (it != ctx->tuning.end()) return it->second;
-  return default_tuning(interp, cls, prec, positions);
+  return g ? job_tuning(interp, cls, prec, positions, g) : default_tuning(interp, cls, prec, positions);
 }
 
 sarbp_status launch(const BpArgs& a, const sarbp_params* p, const sarbp_tuning& t, hipStream_t s) {
@@ -238,7 +240,7 @@ sarbp_status sarbp_backproject(sarbp_context* ctx, const void* d_profiles, const
   if (dg.err != hipSuccess) return hip_fail(dg.err, "hipSetDevice");
   const Fitted fit =
       fit_tuning(get_tuning(ctx, params->interp, params->precision, params->dtype, size_class(grid, params, nullptr),
-                            false),
+                            false, grid),
                  params->precision, grid, params, nullptr);
   BpArgs a;
   st = plan_args(nullptr, grid, params, fit.t, fit.prec, &a, nullptr);
@@ -278,7 +280,7 @@ sarbp_status sarbp_plan_create(sarbp_context* ctx, const double* h_pos, const sa
   }
   const Fitted fit =
       fit_tuning(get_tuning(ctx, params->interp, params->precision, params->dtype, size_class(grid, params, h_pos),
-                            h_pos != nullptr),
+                            h_pos != nullptr, grid),
                  params->precision, grid, params, h_pos);
   const sarbp_tuning& tune = fit.t;
   std::memset(&pl->info, 0, sizeof pl->info);
@@ -381,7 +383,7 @@ sarbp_status sarbp_backproject_batch(sarbp_context* ctx, const sarbp_job* jobs, 
     const sarbp_job& jb = jobs[j];
     if (jb.grid.nx == 0 || jb.grid.ny == 0) continue;
     const Fitted f = fit_tuning(get_tuning(ctx, p0.interp, p0.precision, p0.dtype, size_class(&jb.grid, &jb.params, jb.h_pos),
-                                           jb.h_pos != nullptr),
+                                           jb.h_pos != nullptr, &jb.grid),
                                 p0.precision, &jb.grid, &jb.params, jb.h_pos);
     JobDesc d;
     sarbp_status st = plan_args(jb.h_pos, &jb.grid, &jb.params, f.t, f.prec, &d.a, nullptr, true);
@@ -460,7 +462,7 @@ sarbp_status sarbp_backproject_batch_noalloc(sarbp_context* ctx, const sarbp_job
     const sarbp_job& jb = jobs[order[r]];
     if (jb.grid.nx == 0 || jb.grid.ny == 0) continue;
     const Fitted f = fit_tuning(get_tuning(ctx, p0.interp, p0.precision, p0.dtype, size_class(&jb.grid, &jb.params, jb.h_pos),
-                                           jb.h_pos != nullptr),
+                                           jb.h_pos != nullptr, &jb.grid),
                                 p0.precision, &jb.grid, &jb.params, jb.h_pos);
     JobDesc& d = g_noalloc_plan[n_planned];
     st = plan_args(jb.h_pos, &jb.grid, &jb.params, f.t, f.prec, &d.a, nullptr, true);
@@ -486,7 +488,7 @@ sarbp_status sarbp_backproject_batch_noalloc(sarbp_context* ctx, const sarbp_job
     JobDesc& d = g_noalloc_plan[i];
     d.item_begin = G.items;
     G.items += (int64_t)d.a.tiles_x * d.a.tiles_y;
-    G.shm = std::max(G.shm, lds_layout(G.kinterp, d.a.win, d.a.pulses_per_stage).total);
+    G.shm = std::max(G.shm, launch_lds(d.a));
     ++G.n;
   }
   // Host image of the scratch: headers (counters zero), then each group's
@@ -589,7 +591,7 @@ sarbp_status sarbp_autotune(sarbp_context* ctx, const void* d_profiles, const do
   };
   // default first (built-in, ignoring any stored tuning)
   const int cls = size_class(grid, params, h_pos);
-  const sarbp_tuning def = default_tuning(p.interp, cls, p.precision, h_pos != nullptr);
+  const sarbp_tuning def = job_tuning(p.interp, cls, p.precision, h_pos != nullptr, grid);
   int eff = 0;
   double def_ms = INFINITY;
   st = time_one(def, &def_ms, &eff);

@@ -144,7 +144,7 @@ sarbp_status BatchExec::run(std::vector<JobDesc>& jobs, int interp, int precisio
   for (JobDesc& d : jobs) {
     d.item_begin = items;
     items += (int64_t)d.a.tiles_x * d.a.tiles_y;
-    shm = std::max(shm, lds_layout(interp, d.a.win, d.a.pulses_per_stage).total);
+    shm = std::max(shm, launch_lds(d.a));
   }
   if (items == 0) return SARBP_OK;
   // LDS size class: the largest size (256-B steps) that keeps as many

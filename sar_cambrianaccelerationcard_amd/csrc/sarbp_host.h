@@ -57,6 +57,8 @@ int size_class(const sarbp_grid* g, const sarbp_params* p, const double* h_pos);
 // positions (without them a tile's window covers a disc of its radius, and
 // other tunings win).
 sarbp_tuning default_tuning(int interp, int cls, int precision, bool positions = true);
+// The built-in default of one job: its class's, with taller tiles on large images.
+sarbp_tuning job_tuning(int interp, int cls, int precision, bool positions, const sarbp_grid* g);
 // SARBP_ERR_INVALID_ARGUMENT unless the shape is compiled and 1 <= P <= 256.
 sarbp_status check_tuning(int precision, const sarbp_tuning* t);
 // A tuning fitted to one grid and the arithmetic (kRef, kF64, kF32, kDF) its
@@ -100,6 +102,8 @@ sarbp_status launch(const BpArgs& a, const sarbp_params* p, const sarbp_tuning& 
 struct GroupKey {
   int px, py, kinterp, kprec, occ;
 };
+// Dynamic LDS of a planned launch.
+size_t launch_lds(const BpArgs& a);
 GroupKey group_key(const BpArgs& a, const sarbp_tuning& t, int dtype);
 // Assigns keys[0..n) to groups in first-seen order (group indices to out).
 // Keys that differ only in occ share a group when keeping them apart would

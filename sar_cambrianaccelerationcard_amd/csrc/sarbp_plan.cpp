@@ -218,6 +218,23 @@ sarbp_tuning default_tuning(int interp, int cls, int precision, bool positions) 
   return t;
 }
 
+// The built-in default for one job: on an image of many tiles the continuous
+// interpolators of SARBP_PREC_REF run 64 x 32 instead of 64 x 16 tiles, whose
+// row polynomials and FP64 setup serve twice the pixels.  Below about five
+// rounds of the 1024 workgroups that the chip holds, the coarser work items'
+// last round costs more than that: 1024 pulses over 3584^2 pixels (6272 tiles)
+// ran 4-11% faster at every spacing from 0.25 to 1 m, 2560^2 (3200 tiles)
+// between 2% faster and 5% slower, 1536^2 (1152 tiles) 5-40% slower.
+sarbp_tuning job_tuning(int interp, int cls, int precision, bool positions, const sarbp_grid* g) {
+  sarbp_tuning t = default_tuning(interp, cls, precision, positions);
+  constexpr int64_t kManyTiles = 5 * 1024;
+  const int64_t tiles = (int64_t)((g->nx + 63) / 64) * ((g->ny + 31) / 32);
+  if (precision == SARBP_PREC_REF && interp != SARBP_INTERP_NEAREST && t.cols_per_lane == 1 && t.rows_per_lane == 4 &&
+      tiles >= kManyTiles)
+    t.rows_per_lane = 8;
+  return t;
+}
+
 // Largest |pixel - tile reference| the FP32 differential supports.  Two FP32
 // roundings grow with it: pp = |d|^2 - s^2 carries ~ulp(|d|^2) into
 // q = pp / (2R), a phase error ~ k ulp(|d|^2) / (2R) (at 48 m and R = 5 km,
@@ -435,6 +452,28 @@ double df_quant(const sarbp_grid* g, int px, int py) {
   return std::ldexp(1.0, 23 - (int)std::ceil(std::log2(span)));
 }
 
+size_t launch_lds(const BpArgs& a) {
+  return lds_layout(a.kernel_interp, a.win, a.pulses_per_stage, a.pool).total;
+}
+
+// Positions (sinc8) or samples (linear) that a row-polynomial launch stages
+// at once: the `most` windows of its tuning, or less where that lets one more
+// workgroup share a CU (the kernels' registers allow 4), but never less than
+// one whole window, which a pulse without a bound on its bins needs.  The
+// kernel packs the pulses of a stage at the length they touch, 50-65% of the
+// planned window, so a smaller pool still holds several: 3584^2 x 1024 pulses
+// at 1 m (324-sample windows) ran 31.8 ms with 56 KB of LDS, 23.9 ms with 40;
+// 2560^2 at 0.5 m (104 samples) 7.4 ms with 42.5 KB, 6.7 ms with 40.
+int stage_pool(int kinterp, int win, int P, int most) {
+  const int room = window_room(kinterp, win), bytes = room_bytes(kinterp);
+  const size_t fixed = lds_layout(kinterp, win, P, 16).total - 16 * (size_t)bytes;
+  for (int per_cu = 4; per_cu > 1; --per_cu) {
+    const size_t budget = std::min(kLdsBudget, (kCuLds / per_cu - kBatchStaticLds) & ~(size_t)255);
+    if (fixed + (size_t)room * bytes <= budget) return (int)std::min<size_t>((size_t)most * room, (budget - fixed) / bytes);
+  }
+  return most * room;
+}
+
 // Fills a launch descriptor.  Caller holds ctx->mu and the device guard.
 sarbp_status plan_args(const double* h_pos, const sarbp_grid* g,
                        const sarbp_params* p, const sarbp_tuning& tune, int kprec, BpArgs* a,
@@ -469,11 +508,12 @@ sarbp_status plan_args(const double* h_pos, const sarbp_grid* g,
   // occupancy and fit down to 1 pulse (64 mixed jobs: 191.7 ms that way,
   // 217.0 ms stopping at 4, same box).  The depth changes no result bit:
   // each pixel adds its pulses in pulse order whatever the stages.
-  const int min_stage = batched ? 1 : 4;
   auto per_cu = [&](int q) {
     return kernel_occupancy(kinterp, kprec, p->dtype, px, py, lds_layout(kinterp, win, q).total);
   };
-  while (P > min_stage && per_cu(P - 1) > per_cu(P)) --P;
+  while (P > 4 && per_cu(P - 1) > per_cu(P)) --P;
+  const int plain = P;
+  while (batched && P > 1 && per_cu(P - 1) > per_cu(P)) --P;
 
   std::memset(a, 0, sizeof *a);
   for (int k = 0; k < 3; ++k) {
@@ -506,6 +546,7 @@ sarbp_status plan_args(const double* h_pos, const sarbp_grid* g,
   a->order_tol = 1e-5;
   a->kernel_interp = kinterp;
   a->kernel_prec = kprec;
+  if (kprec == kRef && kinterp != kNearest) a->pool = stage_pool(kinterp, win, P, plain);
   sinc8_kernel_rows(kinterp, p->kaiser_beta, a->sinc_poly);
   if (info) {
     info->tiles_x = a->tiles_x;
@@ -516,7 +557,7 @@ sarbp_status plan_args(const double* h_pos, const sarbp_grid* g,
     info->pulses_per_stage = P;
     info->rows_per_lane = py;
     info->cols_per_lane = px;
-    info->lds_bytes = (int32_t)lds_layout(kinterp, win, P).total;
+    info->lds_bytes = (int32_t)launch_lds(*a);
     info->sinc8_halves = kinterp == kSinc8 ? 2 : (kinterp == kSinc8W ? 1 : 0);
     info->precision = kprec;
     const double rm = ext.rmin > ext.dmax ? ext.rmin - ext.dmax : 0.0;
@@ -528,7 +569,7 @@ sarbp_status plan_args(const double* h_pos, const sarbp_grid* g,
 }
 
 GroupKey group_key(const BpArgs& a, const sarbp_tuning& t, int dtype) {
-  const size_t shm = lds_layout(a.kernel_interp, a.win, a.pulses_per_stage).total;
+  const size_t shm = launch_lds(a);
   int occ = kernel_occupancy(a.kernel_interp, a.kernel_prec, dtype, t.cols_per_lane, t.rows_per_lane, shm);
   if (occ <= 0) occ = (int)std::max<size_t>(1, kCuLds / (shm + kBatchStaticLds));
   return GroupKey{t.cols_per_lane, t.rows_per_lane, a.kernel_interp, a.kernel_prec, occ};

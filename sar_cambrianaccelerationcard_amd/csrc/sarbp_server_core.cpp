@@ -133,6 +133,7 @@ using namespace sarbp;
 struct sarbp_server {
   sarbp_server_config cfg{};
   sarbp_tuning tune[SARBP_SIZE_CLASSES]{};  // per size class; guarded by mu
+  bool tuned[SARBP_SIZE_CLASSES]{};         // not the built-in default; guarded by mu
   int n_cu = 256;
   Arena arena;
   std::mutex mu;
@@ -469,6 +470,7 @@ sarbp_status sarbp::server_create(const sarbp_server_config* cfg, std::unique_pt
     if (cfg->rows_per_lane) t.rows_per_lane = cfg->rows_per_lane;
     if (cfg->cols_per_lane) t.cols_per_lane = cfg->cols_per_lane;
     if (cfg->pulses_per_stage) t.pulses_per_stage = cfg->pulses_per_stage;
+    s->tuned[c] = cfg->rows_per_lane || cfg->cols_per_lane || cfg->pulses_per_stage;
     sarbp_status st = check_tuning(cfg->precision, &t);
     if (st != SARBP_OK) return st;
   }
@@ -519,7 +521,8 @@ sarbp_status sarbp::server_submit(sarbp_server* s, const sarbp_request* req, con
   sarbp_tuning base;
   {
     std::lock_guard<std::mutex> lk(s->mu);
-    base = s->tune[size_class(&req->grid, &p, req->h_pos)];
+    const int cls = size_class(&req->grid, &p, req->h_pos);
+    base = s->tuned[cls] ? s->tune[cls] : job_tuning(p.interp, cls, p.precision, true, &req->grid);
   }
   const Fitted fit = fit_tuning(base, p.precision, &req->grid, &p, req->h_pos);
   j->tune = fit.t;
@@ -569,8 +572,12 @@ sarbp_status sarbp_server_set_class_tuning(sarbp_server* s, int32_t size_cls, co
     v = default_tuning(s->cfg.interp, size_cls, s->cfg.precision);
   sarbp_status st = check_tuning(s->cfg.precision, &v);
   if (st != SARBP_OK) return st;
+  // (a context's untuned class arrives here as the built-in default itself)
+  const sarbp_tuning d = default_tuning(s->cfg.interp, size_cls, s->cfg.precision);
   std::lock_guard<std::mutex> lk(s->mu);
   s->tune[size_cls] = v;
+  s->tuned[size_cls] = v.rows_per_lane != d.rows_per_lane || v.cols_per_lane != d.cols_per_lane ||
+                       v.pulses_per_stage != d.pulses_per_stage;
   return SARBP_OK;
 }
 

@@ -294,3 +294,57 @@ def test_invalid_arguments(ctx, base):
         ctx.backproject(ds.prof.data_ptr(), ds.pos.data_ptr(), g, sc.native_params(), 0)
     with pytest.raises(native.SarbpError):
         ctx.set_tuning(native.INTERP_SINC8, native.PREC_F64, native.DTYPE_C64, 4, 2, 8)  # F64 has cols 1 only
+
+
+@pytest.mark.parametrize("interp", ["linear", "sinc8"])
+@pytest.mark.parametrize("spacing,cols,rows,axes", [
+    (0.1, 1, 2, "xy"), (0.25, 1, 8, "yx"),      # base polynomials, both axis orders
+    (0.7, 1, 8, "xy"), (1.0, 1, 4, "xy"),       # with the x^3 y and y^3 terms
+    (0.25, 4, 4, "skew"), (0.5, 2, 2, "skew"),  # several columns, slanted steps
+    (1.3, 1, 4, "yx"),                          # beyond the polynomials: per pixel
+])
+def test_row_polynomials_match_oracle(base, interp, spacing, cols, rows, axes):
+    """The strip polynomials of REF against the oracle, in every mode, on grids
+    that end inside a tile.  Bound: up to 5e-6 rad of dropped terms, FP32
+    rounding of up to 64 revolutions (2.4e-5 rad), 2e-6 of the sinc8 fit."""
+    sc, ds = base
+    o = sc.grid["origin"]
+    u, v = [spacing, 0.0, 0.0], [0.0, spacing, 0.0]
+    if axes == "yx":
+        u, v = v, u
+    elif axes == "skew":
+        u, v = [0.8 * spacing, 0.5 * spacing, 0.1 * spacing], [-0.4 * spacing, 0.9 * spacing, 0.0]
+    g = {"origin": o, "ux": u, "uy": v, "nx": 70 * cols, "ny": 37}
+    c = native.Context(0)
+    try:
+        c.set_tuning(native.INTERP_NAMES[interp], native.PREC_REF, native.DTYPE_C64, rows, cols, 6)
+        ng = native.make_grid(g["origin"], g["ux"], g["uy"], g["nx"], g["ny"])
+        ref = _oracle(sc, interp, g)
+        for plan in (False, True):
+            img = D.backproject(c, ds, interp=interp, plan=plan, grid=g).cpu().numpy()
+            err = M.rel_l2(img, ref)
+            print(f"  {interp} {spacing} m {cols}x{rows} {axes} plan={plan}: rel_l2={err:.2e} "
+                  f"{c.plan(sc.pos if plan else None, ng, sc.native_params(interp=interp)).info()['precision']}", flush=True)
+            assert err <= 3e-5
+    finally:
+        c.close()
+
+
+def test_antenna_close_to_the_pixels(ctx, base):
+    """Positions a few metres above the grid: no strip has a bound on its bins,
+    every pulse takes the clamped per-pixel form, and pixels right below an
+    antenna hold finite values."""
+    import torch
+    sc, ds = base
+    g = {"origin": [-8.0, -8.0, 0.0], "ux": [0.25, 0, 0], "uy": [0, 0.25, 0], "nx": 64, "ny": 64}
+    pos = sc.pos.copy()
+    pos[:, 0] = np.linspace(-4.0, 4.0, len(pos))
+    pos[:, 1] = 0.0
+    pos[:, 2] = 3.0
+    p = sc.native_params(interp="linear")
+    p.r0 = 0.0
+    d_pos = torch.from_numpy(pos).cuda()
+    img = torch.zeros((64, 64), dtype=torch.complex64, device="cuda")
+    ctx.backproject(ds.prof.data_ptr(), d_pos.data_ptr(), native.make_grid(g["origin"], g["ux"], g["uy"], 64, 64), p,
+                    img.data_ptr(), sync=True)
+    assert np.isfinite(img.cpu().numpy().view(np.float32)).all()
