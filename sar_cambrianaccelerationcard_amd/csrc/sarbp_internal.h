@@ -69,6 +69,8 @@ struct BpArgs {
   int32_t pulse_begin, pulse_end;  // pulses [begin, end) are summed
   int32_t accumulate;
   int32_t pool;           // row polynomials: staged positions (samples) the LDS holds, else 0
+  int32_t parts;          // waves that share a strip's pulses out (1: one workgroup per tile)
+  int32_t sum_pulses;     // pulses per partial sum of a pixel (>= 1)
   int32_t kernel_interp;  // kNearest, kLinear, kSinc8 or kSinc8W
   int32_t kernel_prec;    // kRef, kF64, kF32 or kDF: the arithmetic launched
   // tap-polynomial rows of 4 (sinc8_kernel_rows): kSinc8 [6][P, Q] of the
@@ -99,6 +101,7 @@ __host__ __device__ inline int setup_batch(int P) { return P >= 64 ? P : P * (64
 // two waves' lanes, or one's where a window is long (its pulse records would
 // cost a workgroup per CU), up to the depth of a deep stage.
 __host__ __device__ inline int poly_batch(int P) { return P > 64 ? 64 : (P > 32 ? P : (P >= 4 ? 32 : 16)); }
+constexpr int kMaxParts = 8;             // waves a split strip's pulses are shared out to
 constexpr int kPolyBytes = kWaves * 64;  // records of a pulse's four strips
 
 // LDS layout of one workgroup (byte offsets), SB = setup_batch(P):
@@ -107,17 +110,23 @@ constexpr int kPolyBytes = kWaves * 64;  // records of a pulse's four strips
 //                                 coefficients (float2) of the interpolant at
 //                                 each window position ([2][6] half bins or
 //                                 [8] + 16 B of padding), coef_stride16 x 16 B
-//   par   [SB] 48-B pulse records, or (linear, sinc8) room for the
-//         [poly_batch(P)][4] 64-B strip records of row polynomials
+//   par   [SB] 48-B pulse records
 //   rng   [SB] int2: first staged sample, first sinc8 position of each pulse
 //   start [SB] int window starts
 //   stage [SB/P][3] int per stage: the set of its pulses' range-expansion
 //                   orders (bit o), staged samples and sinc8 positions per
 //                   pulse
-//   tile  [8] double  linear, sinc8: the tile's constants of the setup
-//   pos   [poly_batch(P)][3] double  linear, sinc8: the next batch's positions
 //   poly  [R][4] float  sinc8 only: the tap-polynomial rows (read as
 //                       broadcasts)
+// Row polynomials (pool > 0), NB = poly_batch(P): raw or coef hold `pool`
+// samples or positions in all, and
+//   par   [NB][4] 64-B strip records
+//   pos   [NB][3] double  positions of the next batch
+//   start [NB] int window starts
+//   stage [2][2] int: the set of the strips' modes, positions per pulse
+//   tile  [6] double  the tile's constants of the setup
+// which take no more room at P = 1 than the other layout, so a window that
+// fits one fits both.
 struct LdsLayout {
   size_t raw, coef, par, rng, start, stage, tile, pos, poly, total;
 };
@@ -127,31 +136,35 @@ struct LdsLayout {
 __host__ __device__ constexpr int window_room(int interp, int win) { return sinc_rows(interp) ? win - 7 : win; }
 __host__ __device__ constexpr int room_bytes(int interp) { return sinc_rows(interp) ? coef_stride16(interp) * 16 : 8; }
 
-// pool > 0: room for that many positions or samples in all (row polynomials,
-// which pack the windows at their touched length) instead of P whole windows.
 __host__ __device__ inline LdsLayout lds_layout(int interp, int win, int P, int pool = 0) {
   LdsLayout L;
-  const int SB = setup_batch(P);
-  const size_t room = pool > 0 ? (size_t)pool : (size_t)P * window_room(interp, win);
-  size_t o = 0;
-  L.raw = o;
-  if (sinc_rows(interp) == 0) o += (room * 8 + 15) & ~(size_t)15;  // sinc8 reads its taps from the profile
-  L.coef = o;
-  o += room * coef_stride16(interp) * 16;
+  const int SB = setup_batch(P), NB = poly_batch(P);
+  const size_t staged = (size_t)(pool > 0 ? pool : P * window_room(interp, win)) * room_bytes(interp);
+  size_t o = (staged + 15) & ~(size_t)15;
+  L.raw = L.coef = 0;  // sinc8 reads its taps from the profile
   L.par = o;
-  const size_t par = (size_t)SB * kParBytes, strips = interp == kNearest ? 0 : (size_t)poly_batch(P) * kPolyBytes;
-  o += par > strips ? par : strips;
-  L.rng = o;
-  o += (size_t)SB * 8;
-  L.start = o;
-  o += (size_t)SB * 4;
-  L.stage = o;
-  o += (size_t)(SB / P) * 12;
+  if (pool > 0) {
+    o += (size_t)NB * kPolyBytes;
+    L.pos = o;
+    o += (size_t)NB * 24;
+    L.start = o;
+    o += (size_t)NB * 4;
+    L.stage = o;
+    o += 16;
+    L.tile = o;
+    o += 48;
+    L.rng = o;
+  } else {
+    o += (size_t)SB * kParBytes;
+    L.rng = o;
+    o += (size_t)SB * 8;
+    L.start = o;
+    o += (size_t)SB * 4;
+    L.stage = o;
+    o += (size_t)(SB / P) * 12;
+    L.tile = L.pos = o;
+  }
   o = (o + 15) & ~(size_t)15;
-  L.tile = o;
-  if (interp != kNearest) o += 64;
-  L.pos = o;
-  if (interp != kNearest) o += ((size_t)poly_batch(P) * 24 + 15) & ~(size_t)15;
   L.poly = o;
   o += (size_t)sinc_rows(interp) * 16;
   L.total = (o + 15) & ~(size_t)15;

@@ -11,6 +11,7 @@
 #include <atomic>
 #include <cmath>
 #include <cstdarg>
+#include <cstdint>
 #include <cstdio>
 #include <cstring>
 
@@ -474,6 +475,22 @@ int stage_pool(int kinterp, int win, int P, int most) {
   return most * room;
 }
 
+// Partial sums that a job's pulses are split into, a wave of its strip each:
+// as many as keep the waves within four rounds of the 4096 that the chip
+// holds (256 CUs x 16), with 16 pulses or more in each.  1024 pulses, unsplit
+// against split: 96^2 475 -> 83 us, 512^2 499 -> 281, 768^2 801 -> 630 (sinc8,
+// 0.25 m), 512^2 355 -> 177, 1024^2 727 -> 660 (linear).  A sinc8 strip makes
+// its coefficients alone, where a workgroup per tile shares them among four;
+// from 3072 strips (1024^2 pixels) on that costs more than the split gains:
+// 1041 us unsplit, 1058 split at 0.25 m, 1251 against 1406 at 0.6 m.
+int pulse_parts(int kinterp, int64_t strips, int n_pulses) {
+  constexpr int64_t kWaveRounds = 4 * 4096, kSinc8Strips = 3072;
+  if (kinterp != kLinear && strips > kSinc8Strips) return 1;
+  int parts = 1;
+  while (parts < kMaxParts && strips * parts * 2 <= kWaveRounds && n_pulses >= 32 * parts) parts *= 2;
+  return parts;
+}
+
 // Fills a launch descriptor.  Caller holds ctx->mu and the device guard.
 sarbp_status plan_args(const double* h_pos, const sarbp_grid* g,
                        const sarbp_params* p, const sarbp_tuning& tune, int kprec, BpArgs* a,
@@ -546,7 +563,15 @@ sarbp_status plan_args(const double* h_pos, const sarbp_grid* g,
   a->order_tol = 1e-5;
   a->kernel_interp = kinterp;
   a->kernel_prec = kprec;
-  if (kprec == kRef && kinterp != kNearest) a->pool = stage_pool(kinterp, win, P, plain);
+  a->parts = 1;
+  a->sum_pulses = INT32_MAX;
+  if (kprec == kRef && kinterp != kNearest) {
+    a->pool = stage_pool(kinterp, win, P, plain);
+    if (px == 1) {
+      a->parts = pulse_parts(kinterp, (int64_t)a->tiles_x * a->tiles_y * kWaves, p->n_pulses);
+      if (a->parts > 1) a->sum_pulses = (p->n_pulses + a->parts - 1) / a->parts;
+    }
+  }
   sinc8_kernel_rows(kinterp, p->kaiser_beta, a->sinc_poly);
   if (info) {
     info->tiles_x = a->tiles_x;
