@@ -97,12 +97,21 @@ struct BatchHeader {
 // runs once per SB / P stages.
 __host__ __device__ inline int setup_batch(int P) { return P >= 64 ? P : P * (64 / P); }
 
-// The same for row polynomials, whose setup takes a lane per (pulse, wave):
-// two waves' lanes, or one's where a window is long (its pulse records would
-// cost a workgroup per CU), up to the depth of a deep stage.
-__host__ __device__ inline int poly_batch(int P) { return P > 64 ? 64 : (P > 32 ? P : (P >= 4 ? 32 : 16)); }
-constexpr int kMaxParts = 8;             // waves a split strip's pulses are shared out to
-constexpr int kPolyBytes = kWaves * 64;  // records of a pulse's four strips
+// The launches that image by row polynomials: the continuous interpolators of
+// SARBP_PREC_REF and SARBP_PREC_DF.  16-byte words of their strip records.
+__host__ __device__ constexpr bool row_polynomials(int interp, int prec) {
+  return interp != kNearest && (prec == kRef || prec == kDF);
+}
+__host__ __device__ constexpr int poly_rec16(int prec) { return prec == kDF ? 6 : 4; }
+
+// Their setup batch: a lane per (pulse, wave), of two waves, or of one where a
+// window is long (the records would cost a workgroup per CU), up to the depth
+// of a deep stage; half as many of the longer records.
+__host__ __device__ inline int poly_batch(int P, int rec16) {
+  const int n = P > 64 ? 64 : (P > 32 ? P : (P >= 4 ? 32 : 16));
+  return rec16 > 4 ? n / 2 : n;
+}
+constexpr int kMaxParts = 8;  // waves a split strip's pulses are shared out to
 
 // LDS layout of one workgroup (byte offsets), SB = setup_batch(P):
 //   raw   [P][win] float2         staged range windows (nearest, linear)
@@ -118,9 +127,9 @@ constexpr int kPolyBytes = kWaves * 64;  // records of a pulse's four strips
 //                   pulse
 //   poly  [R][4] float  sinc8 only: the tap-polynomial rows (read as
 //                       broadcasts)
-// Row polynomials (pool > 0), NB = poly_batch(P): raw or coef hold `pool`
+// Row polynomials (pool > 0), NB = poly_batch(P, rec16): raw or coef hold `pool`
 // samples or positions in all, and
-//   par   [NB][4] 64-B strip records
+//   par   [NB][4] strip records of rec16 x 16 B
 //   pos   [NB][3] double  positions of the next batch
 //   start [NB] int window starts
 //   stage [2][2] int: the set of the strips' modes, positions per pulse
@@ -136,15 +145,15 @@ struct LdsLayout {
 __host__ __device__ constexpr int window_room(int interp, int win) { return sinc_rows(interp) ? win - 7 : win; }
 __host__ __device__ constexpr int room_bytes(int interp) { return sinc_rows(interp) ? coef_stride16(interp) * 16 : 8; }
 
-__host__ __device__ inline LdsLayout lds_layout(int interp, int win, int P, int pool = 0) {
+__host__ __device__ inline LdsLayout lds_layout(int interp, int win, int P, int pool = 0, int rec16 = 4) {
   LdsLayout L;
-  const int SB = setup_batch(P), NB = poly_batch(P);
+  const int SB = setup_batch(P), NB = poly_batch(P, rec16);
   const size_t staged = (size_t)(pool > 0 ? pool : P * window_room(interp, win)) * room_bytes(interp);
   size_t o = (staged + 15) & ~(size_t)15;
   L.raw = L.coef = 0;  // sinc8 reads its taps from the profile
   L.par = o;
   if (pool > 0) {
-    o += (size_t)NB * kPolyBytes;
+    o += (size_t)NB * kWaves * rec16 * 16;
     L.pos = o;
     o += (size_t)NB * 24;
     L.start = o;

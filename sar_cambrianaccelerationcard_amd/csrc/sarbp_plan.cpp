@@ -454,7 +454,7 @@ double df_quant(const sarbp_grid* g, int px, int py) {
 }
 
 size_t launch_lds(const BpArgs& a) {
-  return lds_layout(a.kernel_interp, a.win, a.pulses_per_stage, a.pool).total;
+  return lds_layout(a.kernel_interp, a.win, a.pulses_per_stage, a.pool, poly_rec16(a.kernel_prec)).total;
 }
 
 // Positions (sinc8) or samples (linear) that a row-polynomial launch stages
@@ -465,9 +465,9 @@ size_t launch_lds(const BpArgs& a) {
 // planned window, so a smaller pool still holds several: 3584^2 x 1024 pulses
 // at 1 m (324-sample windows) ran 31.8 ms with 56 KB of LDS, 23.9 ms with 40;
 // 2560^2 at 0.5 m (104 samples) 7.4 ms with 42.5 KB, 6.7 ms with 40.
-int stage_pool(int kinterp, int win, int P, int most) {
+int stage_pool(int kinterp, int kprec, int win, int P, int most) {
   const int room = window_room(kinterp, win), bytes = room_bytes(kinterp);
-  const size_t fixed = lds_layout(kinterp, win, P, 16).total - 16 * (size_t)bytes;
+  const size_t fixed = lds_layout(kinterp, win, P, 16, poly_rec16(kprec)).total - 16 * (size_t)bytes;
   for (int per_cu = 4; per_cu > 1; --per_cu) {
     const size_t budget = std::min(kLdsBudget, (kCuLds / per_cu - kBatchStaticLds) & ~(size_t)255);
     if (fixed + (size_t)room * bytes <= budget) return (int)std::min<size_t>((size_t)most * room, (budget - fixed) / bytes);
@@ -480,12 +480,16 @@ int stage_pool(int kinterp, int win, int P, int most) {
 // holds (256 CUs x 16), with 16 pulses or more in each.  1024 pulses, unsplit
 // against split: 96^2 475 -> 83 us, 512^2 499 -> 281, 768^2 801 -> 630 (sinc8,
 // 0.25 m), 512^2 355 -> 177, 1024^2 727 -> 660 (linear).  A sinc8 strip makes
-// its coefficients alone, where a workgroup per tile shares them among four;
-// from 3072 strips (1024^2 pixels) on that costs more than the split gains:
-// 1041 us unsplit, 1058 split at 0.25 m, 1251 against 1406 at 0.6 m.
-int pulse_parts(int kinterp, int64_t strips, int n_pulses) {
-  constexpr int64_t kWaveRounds = 4 * 4096, kSinc8Strips = 3072;
-  if (kinterp != kLinear && strips > kSinc8Strips) return 1;
+// the coefficients of its positions (`room` at most) alone, where a workgroup
+// per tile shares them among four: from 2560 strips or 2^19 positions a pulse
+// on that costs more than the split gains.  Unsplit against split, us, at
+// strips x room: 0.25 m 4096 x 65 1041 / 1058; 0.7 m 2304 x 101 1101 / 905,
+// 3072 x 109 1245 / 1344; 1.25 m 2304 x 213 1603 / 1438, 3072 x 237 1727 /
+// 2432; 1.6 m 1024 x 261 1285 / 887, 2304 x 301 1763 / 2219; 2 m 2304 x 417
+// 2032 / 2847.
+int pulse_parts(int kinterp, int64_t strips, int room, int n_pulses) {
+  constexpr int64_t kWaveRounds = 4 * 4096, kSinc8Strips = 2560, kSinc8Positions = 1 << 19;
+  if (kinterp != kLinear && (strips > kSinc8Strips || strips * room > kSinc8Positions)) return 1;
   int parts = 1;
   while (parts < kMaxParts && strips * parts * 2 <= kWaveRounds && n_pulses >= 32 * parts) parts *= 2;
   return parts;
@@ -565,10 +569,11 @@ sarbp_status plan_args(const double* h_pos, const sarbp_grid* g,
   a->kernel_prec = kprec;
   a->parts = 1;
   a->sum_pulses = INT32_MAX;
-  if (kprec == kRef && kinterp != kNearest) {
-    a->pool = stage_pool(kinterp, win, P, plain);
+  if (row_polynomials(kinterp, kprec)) {
+    a->pool = stage_pool(kinterp, kprec, win, P, plain);
     if (px == 1) {
-      a->parts = pulse_parts(kinterp, (int64_t)a->tiles_x * a->tiles_y * kWaves, p->n_pulses);
+      a->parts = pulse_parts(kinterp, (int64_t)a->tiles_x * a->tiles_y * kWaves, window_room(kinterp, win),
+                             p->n_pulses);
       if (a->parts > 1) a->sum_pulses = (p->n_pulses + a->parts - 1) / a->parts;
     }
   }

@@ -330,6 +330,56 @@ def test_row_polynomials_match_oracle(base, interp, spacing, cols, rows, axes):
         c.close()
 
 
+@pytest.mark.parametrize("interp,spacing,rows,axes", [
+    ("sinc8", 0.4, 2, "xy"), ("sinc8", 1.6, 4, "xy"), ("sinc8", 1.6, 8, "yx"), ("sinc8", 1.9, 2, "skew"),
+    ("linear", 1.0, 2, "yx"), ("linear", 1.6, 8, "xy"), ("linear", 2.4, 4, "skew"),
+    ("linear", 6.0, 2, "xy"),  # beyond the polynomials: FP64 per pixel
+])
+def test_double_float_row_polynomials_match_oracle(base, interp, spacing, rows, axes):
+    """SARBP_PREC_DF on grids that end inside a tile, a workgroup per tile (24
+    pulses) and pulses shared out over waves, against the oracle; the batch
+    gives the planned image's bits.  Bound: 8e-6 rad of dropped terms and FP32
+    rounding of up to 1024 bins (a few of 1.8e-5 bin rms, slope below 1)."""
+    import torch
+    sc, ds = base
+    o = sc.grid["origin"]
+    u, v = [spacing, 0.0, 0.0], [0.0, spacing, 0.0]
+    if axes == "yx":
+        u, v = v, u
+    elif axes == "skew":
+        u, v = [0.8 * spacing, 0.5 * spacing, 0.1 * spacing], [-0.4 * spacing, 0.9 * spacing, 0.0]
+    g = {"origin": o, "ux": u, "uy": v, "nx": 70, "ny": 37}
+    ng = native.make_grid(g["origin"], g["ux"], g["uy"], g["nx"], g["ny"])
+    stream = torch.cuda.current_stream().cuda_stream
+    c = native.Context(0)
+    try:
+        c.set_tuning(native.INTERP_NAMES[interp], native.PREC_DF, native.DTYPE_C64, rows, 1, 4)
+        for pulses in (24, len(sc.pos)):
+            pos = np.ascontiguousarray(sc.pos[:pulses])
+            p = sc.native_params(interp=interp, precision="df")
+            p.n_pulses = pulses
+            ref = O.backproject(np.ascontiguousarray(sc.profiles[:pulses]), pos, g,
+                                O.params(sc.c, sc.fc, sc.r0, sc.dr, interp, sc.kaiser_beta))
+            for h_pos in (None, pos):
+                img = torch.zeros((37, 70), dtype=torch.complex64, device="cuda")
+                pl = c.plan(h_pos, ng, p)
+                assert pl.info()["precision"] == native.PREC_DF
+                pl.execute(ds.prof.data_ptr(), ds.pos.data_ptr(), img.data_ptr(), stream)
+                torch.cuda.synchronize()
+                err = M.rel_l2(img.cpu().numpy(), ref)
+                print(f"  DF {interp} {spacing} m {rows} rows {axes} {pulses} pulses: rel_l2={err:.2e}", flush=True)
+                assert err <= 5e-5
+            jb = native.Job()
+            out = torch.zeros_like(img)
+            jb.d_profiles, jb.d_pos, jb.h_pos = ds.prof.data_ptr(), ds.pos.data_ptr(), pos.ctypes.data
+            jb.grid, jb.params, jb.d_image = ng, p, out.data_ptr()
+            c.backproject_batch([jb], stream)
+            torch.cuda.synchronize()
+            assert np.array_equal(out.cpu().numpy().view(np.uint64), img.cpu().numpy().view(np.uint64))
+    finally:
+        c.close()
+
+
 def test_antenna_close_to_the_pixels(ctx, base):
     """Positions a few metres above the grid: no strip has a bound on its bins,
     every pulse takes the clamped per-pixel form, and pixels right below an
