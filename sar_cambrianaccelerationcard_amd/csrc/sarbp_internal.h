@@ -147,12 +147,12 @@ __host__ __device__ constexpr int room_bytes(int interp) { return sinc_rows(inte
 
 __host__ __device__ inline LdsLayout lds_layout(int interp, int win, int P, int pool = 0, int rec16 = 4) {
   LdsLayout L;
-  const int SB = setup_batch(P), NB = poly_batch(P, rec16);
-  const size_t staged = (size_t)(pool > 0 ? pool : P * window_room(interp, win)) * room_bytes(interp);
-  size_t o = (staged + 15) & ~(size_t)15;
   L.raw = L.coef = 0;  // sinc8 reads its taps from the profile
-  L.par = o;
+  size_t o;
   if (pool > 0) {
+    const int NB = poly_batch(P, rec16);
+    o = ((size_t)pool * room_bytes(interp) + 15) & ~(size_t)15;
+    L.par = o;
     o += (size_t)NB * kWaves * rec16 * 16;
     L.pos = o;
     o += (size_t)NB * 24;
@@ -164,6 +164,9 @@ __host__ __device__ inline LdsLayout lds_layout(int interp, int win, int P, int 
     o += 48;
     L.rng = o;
   } else {
+    const int SB = setup_batch(P);
+    o = (size_t)P * window_room(interp, win) * room_bytes(interp);
+    L.par = o;
     o += (size_t)SB * kParBytes;
     L.rng = o;
     o += (size_t)SB * 8;
