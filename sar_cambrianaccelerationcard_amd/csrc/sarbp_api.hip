@@ -91,14 +91,24 @@ namespace sarbp {
 
 // The context's tuning of a class, else its all-classes tuning, else the
 // built-in default (`positions`: for a plan that knows the antenna positions;
-// `g`: the job's grid, NULL for the class alone).
+// `g`: the job's grid, NULL for the class alone), and whether it is that.
 sarbp_tuning get_tuning(sarbp_context* ctx, int interp, int prec, int dtype, int cls, bool positions = true,
-                        const sarbp_grid* g = nullptr) {
+                        const sarbp_grid* g = nullptr, bool* builtin = nullptr) {
+  if (builtin) *builtin = false;
   auto it = ctx->tuning.find(tuning_key(interp, prec, dtype, cls, positions));
   if (it != ctx->tuning.end()) return it->second;
   it = ctx->tuning.find(tuning_key(interp, prec, dtype, kAllClasses));
   if (it != ctx->tuning.end()) return it->second;
+  if (builtin) *builtin = true;
   return g ? job_tuning(interp, cls, prec, positions, g) : default_tuning(interp, cls, prec, positions);
+}
+
+// The tuning of one job, fitted to its grid.
+Fitted job_fit(sarbp_context* ctx, const sarbp_grid* g, const sarbp_params* p, const double* h_pos) {
+  bool builtin = false;
+  const sarbp_tuning t = get_tuning(ctx, p->interp, p->precision, p->dtype, size_class(g, p, h_pos),
+                                    h_pos != nullptr, g, &builtin);
+  return fit_tuning(t, p->precision, g, p, h_pos, builtin);
 }
 
 sarbp_status launch(const BpArgs& a, const sarbp_params* p, const sarbp_tuning& t, hipStream_t s) {
@@ -238,17 +248,14 @@ sarbp_status sarbp_backproject(sarbp_context* ctx, const void* d_profiles, const
   std::lock_guard<std::mutex> lk(ctx->mu);
   DeviceGuard dg(ctx->device);
   if (dg.err != hipSuccess) return hip_fail(dg.err, "hipSetDevice");
-  const Fitted fit =
-      fit_tuning(get_tuning(ctx, params->interp, params->precision, params->dtype, size_class(grid, params, nullptr),
-                            false, grid),
-                 params->precision, grid, params, nullptr);
+  const Fitted fit = job_fit(ctx, grid, params, nullptr);
   BpArgs a;
-  st = plan_args(nullptr, grid, params, fit.t, fit.prec, &a, nullptr);
+  st = plan_args(nullptr, grid, params, fit.launch, fit.prec, &a, nullptr);
   if (st != SARBP_OK) return st;
   a.prof = d_profiles;
   a.pos = d_pos;
   a.img = reinterpret_cast<float2*>(d_image);
-  return launch(a, params, fit.t, (hipStream_t)stream);
+  return launch(a, params, fit.launch, (hipStream_t)stream);
 }
 
 sarbp_status sarbp_backproject_sync(sarbp_context* ctx, const void* d_profiles, const double* d_pos,
@@ -278,13 +285,11 @@ sarbp_status sarbp_plan_create(sarbp_context* ctx, const double* h_pos, const sa
     delete pl;
     return hip_fail(dg.err, "hipSetDevice");
   }
-  const Fitted fit =
-      fit_tuning(get_tuning(ctx, params->interp, params->precision, params->dtype, size_class(grid, params, h_pos),
-                            h_pos != nullptr, grid),
-                 params->precision, grid, params, h_pos);
-  const sarbp_tuning& tune = fit.t;
+  const Fitted fit = job_fit(ctx, grid, params, h_pos);
   std::memset(&pl->info, 0, sizeof pl->info);
-  st = plan_args(h_pos, grid, params, tune, fit.prec, &pl->args, &pl->info);
+  st = plan_args(h_pos, grid, params, fit.t, fit.prec, &pl->args, &pl->info);
+  if (st == SARBP_OK && fit.launch.rows_per_lane != fit.t.rows_per_lane)
+    st = plan_args(h_pos, grid, params, fit.launch, fit.prec, &pl->args, nullptr);
   if (st != SARBP_OK) {
     delete pl;
     return st;
@@ -293,7 +298,7 @@ sarbp_status sarbp_plan_create(sarbp_context* ctx, const double* h_pos, const sa
   pl->interp = params->interp;
   pl->precision = params->precision;
   pl->dtype = params->dtype;
-  pl->tune = tune;
+  pl->tune = fit.launch;
   *out = pl;
   return SARBP_OK;
 }
@@ -382,19 +387,17 @@ sarbp_status sarbp_backproject_batch(sarbp_context* ctx, const sarbp_job* jobs, 
   for (int32_t j : order) {
     const sarbp_job& jb = jobs[j];
     if (jb.grid.nx == 0 || jb.grid.ny == 0) continue;
-    const Fitted f = fit_tuning(get_tuning(ctx, p0.interp, p0.precision, p0.dtype, size_class(&jb.grid, &jb.params, jb.h_pos),
-                                           jb.h_pos != nullptr, &jb.grid),
-                                p0.precision, &jb.grid, &jb.params, jb.h_pos);
+    const Fitted f = job_fit(ctx, &jb.grid, &jb.params, jb.h_pos);
     JobDesc d;
-    sarbp_status st = plan_args(jb.h_pos, &jb.grid, &jb.params, f.t, f.prec, &d.a, nullptr, true);
+    sarbp_status st = plan_args(jb.h_pos, &jb.grid, &jb.params, f.launch, f.prec, &d.a, nullptr, true);
     if (st != SARBP_OK) return fail(st, "job %d: %s", j, last_detail());
     d.a.prof = jb.d_profiles;
     d.a.pos = jb.d_pos;
     d.a.img = reinterpret_cast<float2*>(jb.d_image);
     d.item_begin = 0;
     planned.push_back(d);
-    tunes.push_back(f.t);
-    keys.push_back(group_key(d.a, f.t, p0.dtype));
+    tunes.push_back(f.launch);
+    keys.push_back(group_key(d.a, f.launch, p0.dtype));
   }
   const int max_groups = (int)(sizeof ctx->batch / sizeof ctx->batch[0]);
   std::vector<int> gid(planned.size());
@@ -461,17 +464,15 @@ sarbp_status sarbp_backproject_batch_noalloc(sarbp_context* ctx, const sarbp_job
   for (int32_t r = 0; r < n_jobs; ++r) {
     const sarbp_job& jb = jobs[order[r]];
     if (jb.grid.nx == 0 || jb.grid.ny == 0) continue;
-    const Fitted f = fit_tuning(get_tuning(ctx, p0.interp, p0.precision, p0.dtype, size_class(&jb.grid, &jb.params, jb.h_pos),
-                                           jb.h_pos != nullptr, &jb.grid),
-                                p0.precision, &jb.grid, &jb.params, jb.h_pos);
+    const Fitted f = job_fit(ctx, &jb.grid, &jb.params, jb.h_pos);
     JobDesc& d = g_noalloc_plan[n_planned];
-    st = plan_args(jb.h_pos, &jb.grid, &jb.params, f.t, f.prec, &d.a, nullptr, true);
+    st = plan_args(jb.h_pos, &jb.grid, &jb.params, f.launch, f.prec, &d.a, nullptr, true);
     if (st != SARBP_OK) return fail(st, "job %d: %s", order[r], last_detail());
     d.a.prof = jb.d_profiles;
     d.a.pos = jb.d_pos;
     d.a.img = reinterpret_cast<float2*>(jb.d_image);
-    tunes[n_planned] = f.t;
-    keys[n_planned] = group_key(d.a, f.t, p0.dtype);
+    tunes[n_planned] = f.launch;
+    keys[n_planned] = group_key(d.a, f.launch, p0.dtype);
     ++n_planned;
   }
   if (n_planned == 0) return SARBP_OK;

@@ -66,14 +66,16 @@ sarbp_status check_tuning(int precision, const sarbp_tuning* t);
 struct Fitted {
   sarbp_tuning t;
   int prec;
+  sarbp_tuning launch;  // t, or its strips cut to two rows (fit_tuning's `builtin`)
 };
 // The tuning with its tile shape reduced, if needed, to the largest compiled
 // shape within it whose tiles fit the REF tile-radius limit on this grid
 // (h_pos, if given, bounds the range from below and relaxes the limit).  A
 // REF job that no shape fits runs the double-float differential (kDF, no
-// radius limit) with one column per lane.
+// radius limit) with one column per lane.  `builtin`: t is the built-in default,
+// whose strips are cut for the launch where the image has few of them.
 Fitted fit_tuning(sarbp_tuning t, int precision, const sarbp_grid* g, const sarbp_params* p,
-                  const double* h_pos);
+                  const double* h_pos, bool builtin = false);
 // Workgroups per CU of the batched BP kernel of interpolator kinterp,
 // arithmetic kprec, profile dtype and tile shape px x py with `shm` bytes of
 // dynamic LDS (registers, LDS and its allocation granularity counted), as the

@@ -303,18 +303,41 @@ double tile_radius(const sarbp_grid* g, int px, int py) {
 int plan_window(const sarbp_grid* g, const sarbp_params* p, int px, int py, const double* h_pos,
                 int* kinterp);
 
+namespace {
+
+// Strips of few rows for an image of few strips, whose pulses go to up to
+// kMaxParts waves a strip: a wave alone on its SIMD takes a strip's rows one
+// after another, ~0.35 us a pulse for two rows and 1.4 for eight, while the
+// chip holds 1024 such waves.  The line lies where two-row strips fill them:
+// 128 four-row strips, 256 where the default tile has eight rows (calls
+// without positions).  1024 pulses, sinc8, eight rows against two: 128^2 180 ->
+// 62 us, 256^2 184 -> 104, 320^2 195 -> 179; four against two: 128^2 82 -> 57,
+// 256 x 128 85 -> 60, 192^2 87 -> 83, 256^2 91 -> 93, 320^2 140 -> 159 (0.25 m);
+// linear 128^2 54 -> 41, 192^2 55 -> 59.  A tile that would be refused is not
+// cut.
+sarbp_tuning cut_strips(sarbp_tuning t, int kprec, const sarbp_grid* g, const sarbp_params* p, const double* h_pos) {
+  const int64_t strips = (int64_t)((g->nx + 63) / 64) * ((g->ny + 15) / 16) * kWaves;  // of four rows
+  if (!row_polynomials(p->interp, kprec) || t.cols_per_lane != 1 || t.rows_per_lane <= 2 ||
+      strips > 32 * std::min(t.rows_per_lane, 8))
+    return t;
+  int kinterp = p->interp;
+  const int win = plan_window(g, p, 1, t.rows_per_lane, h_pos, &kinterp);
+  if (win > 0 && lds_layout(kinterp, win, 1).total <= kLdsBudget) t.rows_per_lane = 2;
+  return t;
+}
+
+// fit_tuning without the cut.
 // The tuning with its tile shape reduced, if needed, to the largest compiled
 // shape no wider and no taller than the requested one whose tiles stay within
 // the radius limit (SARBP_PREC_REF only).  A grid too coarse for every shape
 // runs the double-float differential instead, with one column per lane and
 // the most rows per lane (at most the request's) whose range window fits LDS.
-Fitted fit_tuning(sarbp_tuning t, int precision, const sarbp_grid* g, const sarbp_params* p,
-                  const double* h_pos) {
-  if (precision != SARBP_PREC_REF) return Fitted{t, precision};
+Fitted fit_shape(sarbp_tuning t, int precision, const sarbp_grid* g, const sarbp_params* p, const double* h_pos) {
+  if (precision != SARBP_PREC_REF) return Fitted{t, precision, t};
   auto fits = [&](int px, int py) {
     return tile_radius(g, px, py) <= radius_limit(min_range(g, px, py, h_pos, p->n_pulses), p->dr);
   };
-  if (fits(t.cols_per_lane, t.rows_per_lane)) return Fitted{t, kRef};
+  if (fits(t.cols_per_lane, t.rows_per_lane)) return Fitted{t, kRef, t};
   int best_px = 0, best_py = 0;
   for (int px = t.cols_per_lane; px >= 1; px /= 2)
     for (int py = t.rows_per_lane; py >= 2; py /= 2)
@@ -325,7 +348,7 @@ Fitted fit_tuning(sarbp_tuning t, int precision, const sarbp_grid* g, const sarb
   if (best_px) {
     t.cols_per_lane = best_px;
     t.rows_per_lane = best_py;
-    return Fitted{t, kRef};
+    return Fitted{t, kRef, t};
   }
   t.cols_per_lane = 1;
   int py = std::max(2, std::min(8, t.rows_per_lane));
@@ -336,7 +359,16 @@ Fitted fit_tuning(sarbp_tuning t, int precision, const sarbp_grid* g, const sarb
     py /= 2;
   }
   t.rows_per_lane = py;
-  return Fitted{t, kDF};
+  return Fitted{t, kDF, t};
+}
+
+}  // namespace
+
+Fitted fit_tuning(sarbp_tuning t, int precision, const sarbp_grid* g, const sarbp_params* p, const double* h_pos,
+                  bool builtin) {
+  Fitted f = fit_shape(t, precision, g, p, h_pos);
+  if (builtin) f.launch = cut_strips(f.t, f.prec, g, p, h_pos);
+  return f;
 }
 
 // Range extent (metres, half-width) of one tile seen from any pulse, and the

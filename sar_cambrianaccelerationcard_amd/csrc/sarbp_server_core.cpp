@@ -519,13 +519,15 @@ sarbp_status sarbp::server_submit(sarbp_server* s, const sarbp_request* req, con
   if (!j) return fail(SARBP_ERR_OUT_OF_MEMORY, "job");
   j->req = *req;
   sarbp_tuning base;
+  bool builtin;
   {
     std::lock_guard<std::mutex> lk(s->mu);
     const int cls = size_class(&req->grid, &p, req->h_pos);
+    builtin = !s->tuned[cls];
     base = s->tuned[cls] ? s->tune[cls] : job_tuning(p.interp, cls, p.precision, true, &req->grid);
   }
-  const Fitted fit = fit_tuning(base, p.precision, &req->grid, &p, req->h_pos);
-  j->tune = fit.t;
+  const Fitted fit = fit_tuning(base, p.precision, &req->grid, &p, req->h_pos, builtin);
+  j->tune = fit.launch;
   if ((st = plan_args(req->h_pos, &req->grid, &p, j->tune, fit.prec, &j->args, nullptr, true)) != SARBP_OK)
     return st;
   j->prof_bytes = (size_t)p.n_pulses * p.n_samples * (p.dtype == SARBP_DTYPE_C64 ? 8 : 4);

@@ -70,3 +70,44 @@ def test_split_matches_oracle_and_batch(scene, dtype, interp, pulses, nx, ny, sp
                 assert err <= 3e-5, err
     finally:
         ctx.close()
+
+
+# the default launch cuts strips to two rows up to 128 strips of four rows (256
+# without positions, sinc8): both sides of the line, ragged edges, pixels that
+# take the double-float arithmetic, too few pulses to share out
+@pytest.mark.parametrize("interp,pulses,nx,ny,spacing", [
+    ("sinc8", 301, 100, 250, 0.5), ("sinc8", 301, 100, 260, 0.5), ("sinc8", 40, 129, 300, 0.5), ("sinc8", 20, 65, 17, 1.6),
+    ("linear", 150, 128, 256, 0.5), ("linear", 150, 128, 257, 0.5), ("linear", 64, 30, 33, 2.2),
+])
+def test_small_images_match_oracle_and_batch(scene, interp, pulses, nx, ny, spacing):
+    import torch
+    sc, ds = scene
+    o = sc.grid["origin"]
+    g = {"origin": o, "ux": [spacing, 0.0, 0.0], "uy": [0.0, spacing, 0.0], "nx": nx, "ny": ny}
+    grid = native.make_grid(o, g["ux"], g["uy"], nx, ny)
+    pos = np.ascontiguousarray(sc.pos[:pulses])
+    ref = O.backproject(np.ascontiguousarray(sc.profiles[:pulses]), pos, g,
+                        O.params(sc.c, sc.fc, sc.r0, sc.dr, interp, sc.kaiser_beta))
+    params = sc.native_params(interp=interp)
+    params.n_pulses = pulses
+    stream = torch.cuda.current_stream().cuda_stream
+    ctx = native.Context(0)
+    try:
+        for h_pos in (None, pos):
+            print(f"  {interp} {pulses}p {nx}x{ny} {spacing} m positions={h_pos is not None}", flush=True)
+            img = [torch.zeros((ny, nx), dtype=torch.complex64, device="cuda") for _ in range(3)]
+            ctx.plan(h_pos, grid, params).execute(ds.profiles_ptr("c64"), ds.pos.data_ptr(), img[0].data_ptr(), stream)
+            if h_pos is None:
+                ctx.backproject(ds.profiles_ptr("c64"), ds.pos.data_ptr(), grid, params, img[1].data_ptr(), stream)
+            jb = native.Job()
+            jb.d_profiles, jb.d_pos, jb.d_image = ds.profiles_ptr("c64"), ds.pos.data_ptr(), img[2].data_ptr()
+            jb.h_pos = h_pos.ctypes.data if h_pos is not None else None
+            jb.grid, jb.params = grid, params
+            ctx.backproject_batch([jb], stream)
+            torch.cuda.synchronize()
+            got = [im.cpu().numpy() for im in img]
+            assert M.rel_l2(got[0], ref) <= 5e-5  # bins and phases as in the row polynomials' own tests
+            for other in (got[2],) if h_pos is not None else got[1:]:
+                assert np.array_equal(other.view(np.uint64), got[0].view(np.uint64))
+    finally:
+        ctx.close()
