@@ -244,9 +244,9 @@ const char* sarbp_last_error_detail(void);
  * SARBP_PREC_REF take at most the LDS that lets 4 workgroups share a CU, and
  * pack it with as many pulses as fit at the length they touch.
  * The depth changes no bit of an image.  Where no tuning is set, linear and
- * sinc8 images of at most 32 rows_per_lane strips of 64 x 4 pixels (REF, DF)
- * are launched with 2 rows per lane; sarbp_plan_info describes the tile that
- * the tuning names.  Shapes: rows 2, 4 or 8 with
+ * sinc8 images of few 64 x 4 pixel strips (REF, DF; up to 32 rows_per_lane) are
+ * launched with 2 rows per lane, or (8 rows, up to 640) with 4;
+ * sarbp_plan_info describes the tile that the tuning names.  Shapes: rows 2, 4 or 8 with
  * cols 1 or 2; rows 2 or 4 with cols 4 (SARBP_PREC_REF); cols 1 otherwise. */
 typedef struct sarbp_tuning {
   int32_t rows_per_lane;

@@ -66,7 +66,7 @@ sarbp_status check_tuning(int precision, const sarbp_tuning* t);
 struct Fitted {
   sarbp_tuning t;
   int prec;
-  sarbp_tuning launch;  // t, or its strips cut to two rows (fit_tuning's `builtin`)
+  sarbp_tuning launch;  // t, or its strips cut to fewer rows (fit_tuning's `builtin`)
 };
 // The tuning with its tile shape reduced, if needed, to the largest compiled
 // shape within it whose tiles fit the REF tile-radius limit on this grid

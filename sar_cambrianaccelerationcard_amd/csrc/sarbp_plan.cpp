@@ -225,7 +225,12 @@ sarbp_tuning default_tuning(int interp, int cls, int precision, bool positions) 
 // rounds of the 1024 workgroups that the chip holds, the coarser work items'
 // last round costs more than that: 1024 pulses over 3584^2 pixels (6272 tiles)
 // ran 4-11% faster at every spacing from 0.25 to 1 m, 2560^2 (3200 tiles)
-// between 2% faster and 5% slower, 1536^2 (1152 tiles) 5-40% slower.
+// between 2% faster and 5% slower, 1536^2 (1152 tiles) 5-40% slower.  Without
+// positions the widest windows' 64 x 32 tiles have LDS for fewer workgroups
+// per CU, which shows where there are few tiles: 512 pulses over 1024^2 pixels
+// took 814 / 809 / 1161 / 1229 us by 64 x 32 at 0.7 / 0.8 / 1 / 1.3 m, 672 /
+// 697 / 749 / 1288 by 64 x 16; over 2048^2 2362 / 2592 / 3633 / 4484 against
+// 2464 / 2577 / 3026 / 4405, over 3584^2 64 x 32 wins by 6-18%.
 sarbp_tuning job_tuning(int interp, int cls, int precision, bool positions, const sarbp_grid* g) {
   sarbp_tuning t = default_tuning(interp, cls, precision, positions);
   constexpr int64_t kManyTiles = 5 * 1024;
@@ -233,6 +238,10 @@ sarbp_tuning job_tuning(int interp, int cls, int precision, bool positions, cons
   if (precision == SARBP_PREC_REF && interp != SARBP_INTERP_NEAREST && t.cols_per_lane == 1 && t.rows_per_lane == 4 &&
       tiles >= kManyTiles)
     t.rows_per_lane = 8;
+  constexpr int64_t kFewTiles = 1536;
+  if (precision == SARBP_PREC_REF && interp == SARBP_INTERP_SINC8 && !positions && cls == SARBP_SIZE_CLASSES - 1 &&
+      tiles <= kFewTiles)
+    t.rows_per_lane = 4;
   return t;
 }
 
@@ -313,16 +322,18 @@ namespace {
 // without positions).  1024 pulses, sinc8, eight rows against two: 128^2 180 ->
 // 62 us, 256^2 184 -> 104, 320^2 195 -> 179; four against two: 128^2 82 -> 57,
 // 256 x 128 85 -> 60, 192^2 87 -> 83, 256^2 91 -> 93, 320^2 140 -> 159 (0.25 m);
-// linear 128^2 54 -> 41, 192^2 55 -> 59.  A tile that would be refused is not
-// cut.
+// linear 128^2 54 -> 41, 192^2 55 -> 59.  Up to 640 strips the eight rows are
+// cut to four: 320^2 200 -> 168 us, 384^2 291 -> 238, 512^2 (1024 strips) 326 and
+// 329.  A tile that would be refused is not cut.
 sarbp_tuning cut_strips(sarbp_tuning t, int kprec, const sarbp_grid* g, const sarbp_params* p, const double* h_pos) {
   const int64_t strips = (int64_t)((g->nx + 63) / 64) * ((g->ny + 15) / 16) * kWaves;  // of four rows
-  if (!row_polynomials(p->interp, kprec) || t.cols_per_lane != 1 || t.rows_per_lane <= 2 ||
-      strips > 32 * std::min(t.rows_per_lane, 8))
+  const int rows = t.rows_per_lane == 8 && strips > 256 ? 4 : 2;
+  if (!row_polynomials(p->interp, kprec) || t.cols_per_lane != 1 || t.rows_per_lane <= rows ||
+      strips > (rows == 4 ? 640 : 32 * t.rows_per_lane))
     return t;
   int kinterp = p->interp;
   const int win = plan_window(g, p, 1, t.rows_per_lane, h_pos, &kinterp);
-  if (win > 0 && lds_layout(kinterp, win, 1).total <= kLdsBudget) t.rows_per_lane = 2;
+  if (win > 0 && lds_layout(kinterp, win, 1).total <= kLdsBudget) t.rows_per_lane = rows;
   return t;
 }
 

@@ -73,10 +73,11 @@ def test_split_matches_oracle_and_batch(scene, dtype, interp, pulses, nx, ny, sp
 
 
 # the default launch cuts strips to two rows up to 128 strips of four rows (256
-# without positions, sinc8): both sides of the line, ragged edges, pixels that
-# take the double-float arithmetic, too few pulses to share out
+# without positions, sinc8, and to four up to 640): both sides of the lines,
+# ragged edges, pixels that take the double-float arithmetic, too few pulses to
+# share out
 @pytest.mark.parametrize("interp,pulses,nx,ny,spacing", [
-    ("sinc8", 301, 100, 250, 0.5), ("sinc8", 301, 100, 260, 0.5), ("sinc8", 40, 129, 300, 0.5), ("sinc8", 20, 65, 17, 1.6),
+    ("sinc8", 301, 100, 250, 0.5), ("sinc8", 301, 100, 260, 0.5), ("sinc8", 64, 640, 256, 0.5), ("sinc8", 64, 640, 260, 0.5), ("sinc8", 40, 129, 300, 0.5), ("sinc8", 20, 65, 17, 1.6),
     ("linear", 150, 128, 256, 0.5), ("linear", 150, 128, 257, 0.5), ("linear", 64, 30, 33, 2.2),
 ])
 def test_small_images_match_oracle_and_batch(scene, interp, pulses, nx, ny, spacing):
