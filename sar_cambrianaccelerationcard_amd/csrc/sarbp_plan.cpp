@@ -436,6 +436,7 @@ Extent tile_extent(const sarbp_grid* g, int px, int py, const double* h_pos, int
   }
   const double lux = std::sqrt(uxx), luy = std::sqrt(uyy);
   double amax = 0.0, bmax = 0.0, lo = INFINITY, hi = -INFINITY;
+  int unordered = 0;
   for (int m = 0; m < n_pulses; ++m) {
     const double* a = h_pos + 3 * (size_t)m;
     const double w[3] = {a[0] - g->origin[0], a[1] - g->origin[1], a[2] - g->origin[2]};
@@ -443,11 +444,12 @@ Extent tile_extent(const sarbp_grid* g, int px, int py, const double* h_pos, int
     const double inv = 1.0 / std::fabs(sep);
     lo = sep < lo ? sep : lo;
     hi = sep > hi ? sep : hi;
+    unordered |= sep != sep;
     const double nx_ = std::max(cx[1] - u, u - cx[0]) * inv, ny_ = std::max(cy[1] - v, v - cy[0]) * inv;
     amax = nx_ > amax ? nx_ : amax;
     bmax = ny_ > bmax ? ny_ : bmax;
   }
-  if (!(lo > 0.0) && !(hi < 0.0)) return e;  // antennas on both sides: no bound
+  if (unordered || (!(lo > 0.0) && !(hi < 0.0))) return e;  // NaN, or antennas on both sides: no bound
   amax = std::min(lux, amax);
   bmax = std::min(luy, bmax);
   const double rmin = lo > 0.0 ? lo : -hi;
