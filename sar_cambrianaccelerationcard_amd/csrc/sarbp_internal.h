@@ -145,42 +145,55 @@ struct LdsLayout {
 __host__ __device__ constexpr int window_room(int interp, int win) { return sinc_rows(interp) ? win - 7 : win; }
 __host__ __device__ constexpr int room_bytes(int interp) { return sinc_rows(interp) ? coef_stride16(interp) * 16 : 8; }
 
-__host__ __device__ inline LdsLayout lds_layout(int interp, int win, int P, int pool = 0, int rec16 = 4) {
+__host__ __device__ inline LdsLayout poly_layout(int interp, int P, int pool, int rec16) {
   LdsLayout L;
-  L.raw = L.coef = 0;  // sinc8 reads its taps from the profile
-  size_t o;
-  if (pool > 0) {
-    const int NB = poly_batch(P, rec16);
-    o = ((size_t)pool * room_bytes(interp) + 15) & ~(size_t)15;
-    L.par = o;
-    o += (size_t)NB * kWaves * rec16 * 16;
-    L.pos = o;
-    o += (size_t)NB * 24;
-    L.start = o;
-    o += (size_t)NB * 4;
-    L.stage = o;
-    o += 16;
-    L.tile = o;
-    o += 48;
-    L.rng = o;
-  } else {
-    const int SB = setup_batch(P);
-    o = (size_t)P * window_room(interp, win) * room_bytes(interp);
-    L.par = o;
-    o += (size_t)SB * kParBytes;
-    L.rng = o;
-    o += (size_t)SB * 8;
-    L.start = o;
-    o += (size_t)SB * 4;
-    L.stage = o;
-    o += (size_t)(SB / P) * 12;
-    L.tile = L.pos = o;
-  }
+  L.raw = L.coef = L.rng = 0;
+  const int NB = poly_batch(P, rec16);
+  size_t o = ((size_t)pool * room_bytes(interp) + 15) & ~(size_t)15;
+  L.par = o;
+  o += (size_t)NB * kWaves * rec16 * 16;
+  L.pos = o;
+  o += (size_t)NB * 24;
+  L.start = o;
+  o += (size_t)NB * 4;
+  L.stage = o;
+  o += 16;
+  L.tile = o;
+  o += 48;
   o = (o + 15) & ~(size_t)15;
   L.poly = o;
   o += (size_t)sinc_rows(interp) * 16;
   L.total = (o + 15) & ~(size_t)15;
   return L;
+}
+
+// Two functions, not one with a branch: the kernels evaluate them, and the
+// other form's values cost registers (1 x 4 tiles then spilled: 1024 x 768
+// coarse pixels 3.93 -> 4.28 ms).
+__host__ __device__ inline LdsLayout lds_layout(int interp, int win, int P) {
+  LdsLayout L;
+  L.raw = L.coef = 0;  // sinc8 reads its taps from the profile
+  const int SB = setup_batch(P);
+  size_t o = (size_t)P * window_room(interp, win) * room_bytes(interp);
+  L.par = o;
+  o += (size_t)SB * kParBytes;
+  L.rng = o;
+  o += (size_t)SB * 8;
+  L.start = o;
+  o += (size_t)SB * 4;
+  L.stage = o;
+  o += (size_t)(SB / P) * 12;
+  L.tile = L.pos = o;
+  o = (o + 15) & ~(size_t)15;
+  L.poly = o;
+  o += (size_t)sinc_rows(interp) * 16;
+  L.total = (o + 15) & ~(size_t)15;
+  return L;
+}
+
+// The layout of a launch: `pool` > 0 for row polynomials.
+inline LdsLayout lds_layout(int interp, int win, int P, int pool, int rec16) {
+  return pool > 0 ? poly_layout(interp, P, pool, rec16) : lds_layout(interp, win, P);
 }
 
 // Tile shapes (PX columns x PY rows per lane) with compiled kernels: every
