@@ -71,7 +71,7 @@ def build_sarbp(force: bool = True) -> str:
     srcs = [os.path.join(CSRC, f) for f in SARBP_SOURCES]
     hsrcs = [os.path.join(CSRC, f) for f in SARBP_HOST_SOURCES]
     deps = srcs + hsrcs + [os.path.join(CSRC, h) for h in (
-        "sarbp_internal.h", "sarbp_host.h", "sarbp_fft.h", "sarbp_kernels.inc", "sarbp_rotation.h",
+        "sarbp_internal.h", "sarbp_host.h", "sarbp_fft.h", "sarbp_kernels.inc", "sarbp_rotation.h", "sarbp_poly.h",
         "sarbp_server_core.h")] + [os.path.join(INCLUDE, "sarbp.h")]
     if not force and _newer(out, deps):
         return out

@@ -1,0 +1,285 @@
+// sarbp_poly.h -- row polynomials: the slant range over a wave's strip of pixels
+// as a short polynomial in the pixel offsets, with the bounds that say where it
+// holds.  Plain C++, so that the host tests check the setup that the kernels of
+// sarbp_kernels.inc run.
+#pragma once
+
+#include <math.h>
+#include <string.h>
+
+#include "sarbp_internal.h"
+
+#define SARBP_HD __host__ __device__ inline __attribute__((always_inline))
+
+namespace sarbp {
+
+SARBP_HD float float_of_bits(int v) {
+  float f;
+  memcpy(&f, &v, sizeof f);
+  return f;
+}
+
+// 1 / sqrt(v) to 2^-23 or better.
+SARBP_HD double rsqrt_estimate(double v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_rsq(v);
+#else
+  return (double)(float)(1.0 / sqrt(v));
+#endif
+}
+
+template <int INTERP>
+SARBP_HD constexpr double bin_scale() {
+  return INTERP == kSinc8 ? 2.0 : 1.0;
+}
+
+// ---- row polynomials (SARBP_PREC_REF and _DF, linear and sinc8) -------------------------
+//
+// A wave's pixels of one pulse lie in a strip of 64 PX x PY pixels, over which
+// the slant range is a short polynomial.  With the wave's centre pixel as the
+// expansion point, x the (integer) column offset, y the row offset
+// (half-integer), s = e.d, pp = |d|^2 - s^2 and g = 1 / (2 R0):
+//   R - R0 = s + g pp - 2 g^2 s pp + g^3 (4 s^2 pp - pp^2) + O(d^5 / R0^4)
+//          = s + sum c_ij x^i y^j,   2 <= i + j <= 4.
+// One lane per (pulse, wave) computes the c_ij in FP64; a lane evaluates the
+// terms in x once per pulse and the rows y = +-1/2, +-3/2 .. in pairs, so a
+// pixel costs 3 FMA for its bin and phase together plus 13 / PY operations,
+// where the expansion evaluated per pixel took 10 (order 2).  Terms of fourth
+// and third order that are not kept whole are replaced by their best lower-
+// order fit over the strip (x^3 -> 3/4 X^2 x and the like).
+//   mode 0 keeps x^2 .. x^4, y x, y x^2, y^2, y^2 x;
+//   mode 1 adds y x^3 and y^3;
+//   mode 2 evaluates the exact two-step form per pixel, with its bin clamped.
+// The setup takes the first mode whose dropped terms stay below kPolyTol of
+// phase (mode 2 also where the window bound does not hold, as for antennas
+// among the pixels or positions that are not numbers).
+// 4096 x 4096 x 4096 pulses, 0.25 m, sinc8: 59 ms with the expansion per pixel
+// (36.9 VALU instructions and 28.6 issue slots per pixel-pulse, 1 x 4 pixels
+// per lane), 48.3 ms this way at 1 x 8 (27 in the pixel loop), bound by the
+// VALU issue slots at 84% with the LDS pipe 65% busy beside them.
+constexpr float kPolyTol[2] = {1.5e-6f, 5e-6f};  // rad, modes 0 and 1
+// Record of a (pulse, wave), poly_rec16(PREC) float4:
+// {c0, pa, A2, A3 | A4, pb, B1, B2 | C0, C1, bin0, alpha | beta, B3, D3, tag};
+// phases in revolutions, ranges in bin units.  Mode 2: {c0, pa, 2 R0, last bin
+// | g, pb, 2 g^2, - | -, -, bin0, alpha | beta, -, -, tag} with alpha and beta
+// in m.  tag: the mode in bits 0-1, above them the byte offset of the strip's
+// first position in the pulse's staged ones.
+//
+// SARBP_PREC_DF takes the same expansion further (x^5, y x^3, y x^4, y^2 x^2,
+// y^3) and evaluates the terms that reach tens of revolutions, pa x + a2 x^2,
+// without rounding: pa and a2 are split into multiples of 2^-17, whose products
+// with the integers x and x^2 and their sum are exact in FP32 and lose their
+// whole revolutions exactly, and FP32 remainders.  The phase is then good to
+// ~4e-7 rad rms (1.5e-6 at most) up to 2 m pixels at 5 km, against 1.4e-6 rms
+// of the double-float form per pixel.  Where the dropped terms exceed
+// kCompTol, or without a bound, every pixel's range and phase are FP64 (mode
+// 2).  1024 x 768 pixels of 1.6 m, 2048 pulses, sinc8: 6.95 ms per pixel in
+// double-float, 3.9 by rows.
+// Record: {c0, pa hi, pa lo, a2 hi | a2 lo, A2, A3, A4 | A5, pb, B1, B2 |
+// B3, B4, C0, C1 | C2, D3, bin0, alpha | beta, last bin, -, tag}.  Mode 2:
+// {antenna x, y (FP64) | z, range of the first position (FP64) | .. | -, last
+// bin, -, tag}.
+constexpr float kCompTol = 8e-6f;  // rad, a bound: at it the error is ~1.2e-6 rms
+constexpr double kCompGrid = 131072.0;
+
+// Largest bin (the interpolator's unit) of n staged positions or samples.
+template <int INTERP>
+SARBP_HD constexpr int bin_last(int n) {
+  return INTERP == kSinc8 ? 2 * n - 1 : (INTERP == kSinc8W ? n - 1 : n - 2);
+}
+// The setup's per-launch constants, opaque at each use: what is computed from
+// them alone (S, FP32 copies) is made again per batch instead of being held in
+// registers through the pixel loop, which spilled 11 of them.
+struct SetupArgs {
+  double inv_dr, k_rev, r0, dmax;
+  int half, win;
+  SARBP_HD explicit SetupArgs(const BpArgs& a)
+      : inv_dr(a.inv_dr), k_rev(a.k_rev), r0(a.r0), dmax(a.dmax), half(a.half), win(a.win) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+s"(inv_dr), "+s"(k_rev), "+s"(r0), "+s"(dmax), "+s"(half), "+s"(win));
+#endif
+  }
+};
+
+// Geometry of one pulse over a wave's strip and its expansion: FP64 where a
+// term is large against the phase tolerance, FP32 for the terms of third order
+// and above (at most a few revolutions over a strip).
+template <int INTERP, int PREC, int PX, int PY>
+struct PolySetup {
+  static constexpr float X = kTileX * PX / 2, Y = 0.5f * (PY - 1);
+  double R0, inv, al, be;  // centre range, 1 / R0, e.ux, e.uy
+  double bin0;             // the centre's bin in the profile
+  double c20;              // x^2 coefficient
+  float alf, bef, a20, a11, a02, g2, g3, c31, c22, c03;
+  float c50, c41;          // SARBP_PREC_DF
+  bool bounded;            // the strip's bins are known and inside the planned window
+  int first, n;            // the n positions (linear: samples) its pixels touch, from bin `first`
+  int mode;
+
+  // (wx, wy, wz): the strip's centre, yc rows from the tile reference pixel;
+  // tc: {-, -, -, |ux|^2, ux.uy, |uy|^2}
+  SARBP_HD PolySetup(const BpArgs& a, double wx, double wy, double wz, double yc, const double* tc,
+                                       const double* pos) {
+    // every kernel that images a job has to round this alike
+#pragma clang fp contract(off)
+    const SetupArgs c(a);
+    const double ex = wx - pos[0], ey = wy - pos[1], ez = wz - pos[2];
+    // 1 / R0 by Newton from the hardware's estimate, then R0 = R^2 / R0 with
+    // its own correction: both to an ulp or two
+    const double r2 = fma(ez, ez, fma(ey, ey, ex * ex));
+    double y = rsqrt_estimate(r2);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const double h = 0.5 * y;
+      y = fma(h, fma(-r2 * y, y, 1.0), y);
+    }
+    const double r = r2 * y;
+    R0 = fma(0.5 * y, fma(-r, r, r2), r);
+    inv = y;
+    al = fma(ez, a.ux[2], fma(ey, a.ux[1], ex * a.ux[0])) * inv;
+    be = fma(ez, a.uy[2], fma(ey, a.uy[1], ex * a.uy[0])) * inv;
+    bin0 = (R0 - c.r0) * c.inv_dr;
+    alf = (float)al;
+    bef = (float)be;
+    // R is convex in d: R0 + s <= R <= R0 + s + |d|^2 / (2 (R0 + s)), and s is
+    // extremal at the strip's corners (the FP32 rounding of the offsets is
+    // inside the margin of one bin)
+    const float smin = fminf(-alf * X, alf * (X - 1.0f)) - fabsf(bef) * Y;
+    const float smax = fmaxf(-alf * X, alf * (X - 1.0f)) + fabsf(bef) * Y;
+    const float r0f = (float)R0, xlo = r0f + smin, dmax = (float)c.dmax;
+    const float up = smax + dmax * dmax / (2.0f * xlo);
+    const double ulo = fma((double)smin, c.inv_dr, bin0);
+    const double uhi = fma((double)up, c.inv_dr, bin0);
+    // The strip's positions have to lie inside the window that whole_window
+    // gives the pulse (a.half bins below the tile reference pixel's): strips
+    // decide one by one, alike in every kernel, and whatever they decide, a
+    // tile's four never span more than that window.  `ref`: the reference
+    // pixel's range from R0, by its difference of squares.  The tenth of a bin
+    // covers the FP32 rounding here.
+    constexpr int kOff = sinc_rows(INTERP) > 0 ? 3 : 0, kEnd = sinc_rows(INTERP) > 0 ? 2 : 3;
+    const float ycf = (float)yc, inv_drf = (float)c.inv_dr;
+    const float m = fmaf(ycf * ycf, (float)tc[5], -2.0f * ycf * bef * r0f);
+    const float ref = m / (r0f + sqrtf(fmaf(r0f, r0f, m)));
+    const bool inside = (smin - ref) * inv_drf >= (float)(kOff + 2 - c.half) + 0.1f &&
+                        (up - ref) * inv_drf <= (float)(kOff + window_room(INTERP, c.win) - c.half - kEnd - 1) - 0.1f;
+    bounded = inside && xlo > 0.5f * r0f && fabs(ulo) < 1.0e9 && fabs(uhi) < 1.0e9;
+    // one bin of margin for the FP32 rounding of a pixel's bin; linear reads
+    // one sample above it
+    first = bounded ? (int)floor(ulo) - 1 : 0;
+    n = bounded ? (int)floor(uhi) - first + (sinc_rows(INTERP) > 0 ? 2 : 3) : 0;
+    const float uxx = (float)tc[3], uyy = (float)tc[5], invf = (float)inv;
+    const double d20 = fma(-al, al, tc[3]);
+    c20 = 0.5 * inv * d20;
+    a20 = (float)d20;
+    a11 = (float)(2.0 * (tc[4] - al * be));
+    a02 = (float)(tc[5] - be * be);
+    g2 = 0.5f * invf * invf;
+    g3 = 0.25f * g2 * invf;
+    c31 = g3 * (4.0f * alf * (alf * a11 + 2.0f * bef * a20) - 2.0f * a20 * a11);
+    c22 = g3 * (4.0f * (alf * alf * a02 + bef * (2.0f * alf * a11 + bef * a20)) - 2.0f * a20 * a02 - a11 * a11);
+    c03 = -g2 * bef * a02;
+    const float lx = X * sqrtf(uxx), ly = Y * sqrtf(uyy), mu = fabsf(alf) * X / lx;
+    const float q1 = lx * invf, q2 = q1 * q1, q4 = q2 * q2;
+    const float rad = 6.2831853f * (float)c.k_rev;
+    if constexpr (PREC == kDF) {
+      const float r4 = 4.0f * g2 * g2;
+      const float af2 = alf * alf;
+      c50 = r4 * alf * a20 * (0.375f * a20 - 0.5f * af2);
+      c41 = r4 * (0.375f * a20 * (bef * a20 + 2.0f * alf * a11) - 0.5f * af2 * (alf * a11 + 3.0f * bef * a20));
+      // dropped: y^3 x and y^4, the fifth order's y^2 x^3 (up to 4 (mu + mu^3))
+      // and y^3 x^2, the sixth's x^6 and y x^5
+      const float c13 = g3 * (4.0f * bef * (bef * a11 + 2.0f * alf * a02) - 2.0f * a11 * a02);
+      const float mu2 = mu * mu;
+      const float e6 = q1 * (lx * (0.0625f + 0.75f * mu2 + 0.5f * mu2 * mu2) + ly * (0.375f + 1.5f * mu));
+      const float e5 = ly * ly / lx * (4.0f * (mu + mu * mu2) + 0.6f * ly / lx);
+      const float e4 = Y * Y * Y * (X * fabsf(c13) + 4.0f * Y * g3 * bef * bef * a02);
+      mode = bounded && rad * (q4 * (e5 + e6) + e4) <= kCompTol ? 0 : 2;
+    } else {
+      // fifth order: (3 mu - 10 mu^3 + 7 mu^5) / 8 of (d / R0)^5 R0 along x, mu
+      // its cosine, and up to 1 of the mixed term; sixth order: up to 1/2
+      const float e5 = q4 * ((0.375f * mu + 1.25f * mu * mu * mu) * lx + ly + 0.5f * lx * q1);
+      const float e22 = 0.5f * X * X * Y * Y * fabsf(c22);
+      const float e31 = 0.25f * X * X * X * Y * fabsf(c31), e03 = 0.25f * Y * Y * Y * fabsf(c03);
+      const float err1 = rad * (e5 + e22), err0 = err1 + rad * (e31 + e03);
+      mode = !bounded ? 2 : (err0 <= kPolyTol[0] ? 0 : (err1 <= kPolyTol[1] ? 1 : 2));
+    }
+  }
+
+  // Where the strip is not bounded: the planned window about the tile reference
+  // pixel, every pixel's bin clamped into it.
+  SARBP_HD void whole_window(const BpArgs& a, const double* tc, const double* pos) {
+    const double ex = tc[0] - pos[0], ey = tc[1] - pos[1], ez = tc[2] - pos[2];
+    const double bc = floor((sqrt(ex * ex + ey * ey + ez * ez) - a.r0) * a.inv_dr) - (double)a.half;
+    first = (int)fmax(fmin(bc, 2.0e9), -2.0e9) + (sinc_rows(INTERP) > 0 ? 3 : 0);
+    n = window_room(INTERP, a.win);
+    mode = 2;
+  }
+
+  // The record of a strip whose positions begin `offset` bytes into the
+  // pulse's staged ones; bins count from `first`.
+  SARBP_HD void store(const BpArgs& a, const double* pos, int offset, float4* r) const {
+#pragma clang fp contract(off)
+    const SetupArgs c(a);
+    constexpr double kS = bin_scale<INTERP>();
+    const float S = (float)(c.inv_dr * kS);
+    // Phase increments per pixel reduced to one revolution, exact for the
+    // integer x; y is half-integer, so the whole revolutions of a row step
+    // leave (PY - 1) / 2 of themselves in the constant.
+    double pa = c.k_rev * al;
+    pa -= rint(pa);
+    double pb = c.k_rev * be;
+    const double turns = rint(pb);
+    pb -= turns;
+    double c0 = fma(c.k_rev, R0, -turns * (0.5 * (PY - 1)));
+    c0 -= floor(c0);
+    const float b0 = (float)(kS * (bin0 - (double)first));
+    const float tag = float_of_bits((offset << 2) | mode);
+    const float g = (float)(0.5 * inv);
+    if constexpr (PREC == kDF) {
+      if (mode == 2) {
+        double* d = reinterpret_cast<double*>(r);
+        for (int k = 0; k < 3; ++k) d[k] = pos[k];
+        d[3] = fma((double)first, a.dr, c.r0);
+        r[5] = make_float4(0.0f, (float)bin_last<INTERP>(n), 0.0f, tag);
+        return;
+      }
+      const double a2 = c.k_rev * c20;
+      const double pah = rint(pa * kCompGrid) * (1.0 / kCompGrid), a2h = rint(a2 * kCompGrid) * (1.0 / kCompGrid);
+      r[0] = make_float4((float)c0, (float)pah, (float)(pa - pah), (float)a2h);
+      r[1] = make_float4((float)(a2 - a2h), (float)(c.inv_dr * kS * c20), -S * g2 * alf * a20,
+                         S * g3 * a20 * (4.0f * alf * alf - a20));
+      r[2] = make_float4(S * c50, (float)pb, S * g * a11, -S * g2 * (alf * a11 + bef * a20));
+      r[3] = make_float4(S * c31, S * c41, S * g * a02, -S * g2 * (alf * a02 + bef * a11));
+      r[4] = make_float4(S * c22, (float)c.k_rev * c03, b0, (float)(c.inv_dr * kS * al));
+      r[5] = make_float4((float)(c.inv_dr * kS * be), (float)bin_last<INTERP>(n), 0.0f, tag);
+      return;
+    }
+    if (mode == 2) {
+      r[0] = make_float4((float)c0, (float)pa, (float)(2.0 * R0), (float)bin_last<INTERP>(n));
+      r[1] = make_float4(g, (float)pb, g2, 0.0f);
+      r[2] = make_float4(0.0f, 0.0f, b0, alf);
+      r[3] = make_float4(bef, 0.0f, 0.0f, tag);
+      return;
+    }
+    // mode 0: x^3 y and y^3 as their best fits in x y and y
+    const float f11 = mode == 0 ? 0.75f * X * X * c31 : 0.0f, f01 = mode == 0 ? 0.75f * Y * Y * c03 : 0.0f;
+    r[0] = make_float4((float)c0, (float)pa, (float)(c.inv_dr * kS * c20), -S * g2 * alf * a20);
+    r[1] = make_float4(S * g3 * a20 * (4.0f * alf * alf - a20), (float)pb + (float)c.k_rev * f01,
+                       S * (g * a11 + f11), -S * g2 * (alf * a11 + bef * a20));
+    r[2] = make_float4(S * (g * a02 + 0.5f * X * X * c22), -S * g2 * (alf * a02 + bef * a11), b0,
+                       (float)(c.inv_dr * kS * al));
+    r[3] = make_float4((float)(c.inv_dr * kS * be) + S * f01, S * c31, (float)c.k_rev * c03, tag);
+  }
+};
+
+// The setup's constants of one tile: its reference pixel and the grid steps'
+// products (kept in LDS, not in 12 registers through the pixel loop).
+SARBP_HD void tile_constants(const BpArgs& a, int x0, int y0, int tx, int ty, double* tc) {
+  const int ic = x0 + tx / 2, jc = y0 + ty / 2;
+  for (int k = 0; k < 3; ++k) tc[k] = a.origin[k] + ic * a.ux[k] + jc * a.uy[k];
+  tc[3] = a.ux[0] * a.ux[0] + a.ux[1] * a.ux[1] + a.ux[2] * a.ux[2];
+  tc[4] = a.ux[0] * a.uy[0] + a.ux[1] * a.uy[1] + a.ux[2] * a.uy[2];
+  tc[5] = a.uy[0] * a.uy[0] + a.uy[1] * a.uy[1] + a.uy[2] * a.uy[2];
+}
+
+}  // namespace sarbp
