@@ -195,13 +195,18 @@ struct PolySetup {
       const float e4 = Y * Y * Y * (X * fabsf(c13) + 4.0f * Y * g3 * bef * bef * a02);
       mode = bounded && rad * (q4 * (e5 + e6) + e4) <= kCompTol ? 0 : 2;
     } else {
-      // fifth order: (3 mu - 10 mu^3 + 7 mu^5) / 8 of (d / R0)^5 R0 along x, mu
-      // its cosine, and up to 1 of the mixed term; sixth order: up to 1/2
-      const float e5 = q4 * ((0.375f * mu + 1.25f * mu * mu * mu) * lx + ly + 0.5f * lx * q1);
-      const float e22 = 0.5f * X * X * Y * Y * fabsf(c22);
+      // Dropped: x y^3 and y^4 whole; x^2 y^2, x^3 y and y^3 but for their fits;
+      // the fifth order, (3 mu - 10 mu^3 + 7 mu^5) / 8 of lx^5 / R0^4 along x
+      // (mu its cosine), off it up to ly times the form's largest gradient, 0.42
+      // |d|^4 / R0^4; and from the sixth on |d| (d / R0)^5 / 16 / (1 - d / R0).
+      const float c13 = g3 * (4.0f * bef * (bef * a11 + 2.0f * alf * a02) - 2.0f * a11 * a02);
+      const float c04 = g3 * a02 * (4.0f * bef * bef - a02);
+      const float l = lx + ly, q = l * invf, ql4 = q * q * q * q;
+      const float e5 = q4 * (0.375f * mu + 1.25f * mu * mu * mu) * lx + ql4 * (0.42f * ly + 0.125f * q * l);
+      const float e4 = Y * Y * (0.5f * X * X * fabsf(c22) + X * Y * fabsf(c13) + Y * Y * fabsf(c04));
       const float e31 = 0.25f * X * X * X * Y * fabsf(c31), e03 = 0.25f * Y * Y * Y * fabsf(c03);
-      const float err1 = rad * (e5 + e22), err0 = err1 + rad * (e31 + e03);
-      mode = !bounded ? 2 : (err0 <= kPolyTol[0] ? 0 : (err1 <= kPolyTol[1] ? 1 : 2));
+      const float err1 = rad * (e5 + e4), err0 = err1 + rad * (e31 + e03);
+      mode = !(bounded && q <= 0.5f) ? 2 : (err0 <= kPolyTol[0] ? 0 : (err1 <= kPolyTol[1] ? 1 : 2));
     }
   }
 

@@ -5,6 +5,8 @@
 //   window   every strip's staged positions lie inside the pulse's planned
 //            window, whatever the antenna positions, and a bounded strip's hold
 //            every pixel's bin with half a bin to spare.
+//   ref      SARBP_PREC_REF: what the accepted mode leaves out stays within its
+//            tolerance, for pixels of any shape (aspect 1:100 to 100:1).
 // Exit status 0 when the named check passes.
 #include <algorithm>
 #include <cmath>
@@ -153,11 +155,168 @@ void check_window() {
         g_strips);
 }
 
+// Kept terms of R - R0 (long double) of a strip: the Taylor expansion of
+// sqrt((R0 + s)^2 + pp) in (s, pp) up to `fourth` order whole, its monomials
+// x^i y^j of third order and above filtered by keep(i, j) -> factor on another
+// monomial.  Coefficients c[i][j] by expanding the powers of s and pp.
+struct Series {
+  long double c[8][8] = {};  // c[i][j] x^i y^j, total degree <= 6
+};
+using Poly = Series;
+Poly mul(const Poly& a, const Poly& b) {
+  Poly r;
+  for (int i = 0; i < 7; ++i)
+    for (int j = 0; i + j < 7; ++j)
+      if (a.c[i][j] != 0)
+        for (int k = 0; i + j + k < 7; ++k)
+          for (int l = 0; i + j + k + l < 7; ++l) r.c[i + k][j + l] += a.c[i][j] * b.c[k][l];
+  return r;
+}
+Poly add(const Poly& a, const Poly& b, long double f) {
+  Poly r = a;
+  for (int i = 0; i < 8; ++i)
+    for (int j = 0; j < 8; ++j) r.c[i][j] += f * b.c[i][j];
+  return r;
+}
+
+// Strip geometry in long double.
+struct Exact {
+  long double R0, al, be, uxx, uxy, uyy;
+  Exact(const BpArgs& a, const double* centre, const double* pos) {
+    long double e[3], r2 = 0;
+    al = be = uxx = uxy = uyy = 0;
+    for (int k = 0; k < 3; ++k) e[k] = (long double)centre[k] - pos[k], r2 += e[k] * e[k];
+    R0 = sqrtl(r2);
+    for (int k = 0; k < 3; ++k) {
+      al += e[k] * a.ux[k] / R0;
+      be += e[k] * a.uy[k] / R0;
+      uxx += (long double)a.ux[k] * a.ux[k];
+      uxy += (long double)a.ux[k] * a.uy[k];
+      uyy += (long double)a.uy[k] * a.uy[k];
+    }
+  }
+  // R - R0 at (x, y), without cancellation
+  long double at(long double x, long double y) const {
+    const long double s = al * x + be * y, dd = uxx * x * x + 2 * uxy * x * y + uyy * y * y;
+    const long double t = 2 * R0 * s + dd;
+    return t / (R0 + sqrtl(R0 * R0 + t));
+  }
+  // R - R0 to sixth order
+  Poly series() const {
+    Poly s, pp, one;
+    one.c[0][0] = 1;
+    s.c[1][0] = al, s.c[0][1] = be;
+    pp.c[2][0] = uxx - al * al, pp.c[1][1] = 2 * (uxy - al * be), pp.c[0][2] = uyy - be * be;
+    // sqrt(1 + z), z = (2 R0 s + s^2 + pp) / R0^2, to z^6
+    Poly z = add(add(Poly{}, s, 2 / R0), add(mul(s, s), pp, 1), 1 / (R0 * R0)), zp = one, r;
+    long double b = 1;
+    for (int k = 1; k <= 6; ++k) {
+      zp = mul(zp, z);
+      b *= (1.5L - k) / k;
+      r = add(r, zp, R0 * b);
+    }
+    return r;
+  }
+};
+
+double eval(const Poly& p, double x, double y) {
+  long double r = 0;
+  for (int i = 7; i >= 0; --i) {
+    long double t = 0;
+    for (int j = 7; j >= 0; --j) t = t * y + p.c[i][j];
+    r = r * x + t;
+  }
+  return (double)r;
+}
+
+// A strip of PX x PY pixels per lane at range R: pixels of any shape and slant,
+// a window that holds it.
+template <int PX, int PY>
+void random_strip(Rng& rng, BpArgs& a, double* tc, double* pos, double lx_max, double r_lo, double r_hi) {
+  std::memset(&a, 0, sizeof a);
+  const double R = log_uniform(rng, r_lo, r_hi);
+  const double fc[] = {0.4e9, 1.3e9, 5.3e9, 9.6e9, 35e9};
+  a.k_rev = 2 * fc[rng() % 5] / 299792458.0;
+  const double aspect = log_uniform(rng, 0.01, 100.0), size = log_uniform(rng, 1e-4, 0.3) * R;
+  const double ly_over_lx = (PY - 1) * aspect / (64.0 * PX);
+  double lx = size / std::max(1.0, ly_over_lx);
+  lx = std::min(lx, lx_max);
+  const double sx = lx / (32.0 * PX), sy = sx * aspect, ang = uniform(rng, 0, 6.2831853),
+               slant = uniform(rng, -0.5, 0.5) * (rng() % 2);
+  a.ux[0] = sx * std::cos(ang), a.ux[1] = sx * std::sin(ang);
+  a.uy[0] = -sy * std::sin(ang + slant), a.uy[1] = sy * std::cos(ang + slant);
+  if (rng() % 2) a.ux[2] = sx * uniform(rng, -0.3, 0.3), a.uy[2] = sy * uniform(rng, -0.3, 0.3);
+  const double el = rng() % 4 ? uniform(rng, 0.1, 1.5) : uniform(rng, 0, 0.1), az = rng() % 2 ? 0.0 : uniform(rng, -1.5, 1.5);
+  const double d[3] = {std::cos(el) * std::sin(az), std::cos(el) * std::cos(az), std::sin(el)};
+  tile_constants(a, 0, 0, 0, 0, tc);
+  for (int k = 0; k < 3; ++k) pos[k] = -d[k] * R;
+  const double l = 32.0 * PX * std::sqrt(tc[3]) + 4.0 * PY * std::sqrt(tc[5]);
+  a.dmax = l;
+  a.dr = log_uniform(rng, 1.0, 100.0) * l / 1000;
+  a.inv_dr = 1 / a.dr;
+  a.r0 = R - 100 * a.dr;
+  a.win = 8192;
+  a.half = 4095;
+}
+
+long g_taken[3];
+double g_worst = 0;
+
+template <int PX, int PY>
+void ref_one(Rng& rng) {
+  BpArgs a;
+  double tc[6], pos[3];
+  random_strip<PX, PY>(rng, a, tc, pos, 512.0, 100.0, 8e5);
+  PolySetup<kSinc8, kRef, PX, PY> ps(a, tc[0], tc[1], tc[2], 0.0, tc, pos);
+  ++g_strips;
+  g_bounded += ps.bounded;
+  ++g_taken[ps.mode];
+  if (ps.mode == 2) return;
+  const Exact ex(a, tc, pos);
+  Poly p = ex.series();
+  const double X = 32.0 * PX, Y = 0.5 * (PY - 1);
+  for (int i = 0; i < 7; ++i)
+    for (int j = 0; i + j < 7; ++j) {
+      const long double c = p.c[i][j];
+      const int n = i + j;
+      bool keep = n <= 3 || (n == 4 && j <= 1);
+      if (i == 2 && j == 2) p.c[0][2] += 0.5 * X * X * c;
+      if (ps.mode == 0 && i == 3 && j == 1) p.c[1][1] += 0.75 * X * X * c, keep = false;
+      if (ps.mode == 0 && i == 0 && j == 3) p.c[0][1] += 0.75 * Y * Y * c, keep = false;
+      if (!keep) p.c[i][j] = 0;
+    }
+  double worst = 0;
+  for (int n = 0; n < PY; ++n)
+    for (int k = 0; k <= 16; ++k) {
+      const double x = -X + k * (2 * X - 1) / 16, y = n - Y;
+      worst = std::max(worst, std::fabs((double)ex.at(x, y) - eval(p, x, y)));
+    }
+  const double rad = worst * 6.283185307179586 * a.k_rev;
+  g_worst = std::max(g_worst, rad / kPolyTol[ps.mode]);
+  CHECK(rad <= 1.001 * kPolyTol[ps.mode],
+        "PX %d PY %d mode %d: %.3g rad left out, |ux| %.3g |uy| %.3g R %.4g fc %.3g", PX, PY, ps.mode, rad,
+        std::sqrt(tc[3]), std::sqrt(tc[5]), (double)ex.R0, a.k_rev * 1.5e8);
+}
+
+void check_ref() {
+  Rng rng(11);
+  for (int i = 0; i < 60000; ++i) {
+    ref_one<1, 2>(rng), ref_one<1, 4>(rng), ref_one<1, 8>(rng);
+    ref_one<2, 2>(rng), ref_one<2, 4>(rng), ref_one<2, 8>(rng);
+    ref_one<4, 2>(rng), ref_one<4, 4>(rng);
+  }
+  // every mode is taken, and the bounds are of the errors' size
+  for (long n : g_taken) CHECK(n > g_strips / 100, "modes taken %ld %ld %ld", g_taken[0], g_taken[1], g_taken[2]);
+  CHECK(g_worst > 0.5, "largest error %.2f of the tolerance", g_worst);
+  std::printf("modes %ld %ld %ld, largest error %.2f of the tolerance\n", g_taken[0], g_taken[1], g_taken[2], g_worst);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const char* name = argc > 1 ? argv[1] : "";
   if (!std::strcmp(name, "window")) check_window();
+  else if (!std::strcmp(name, "ref")) check_ref();
   else return std::fprintf(stderr, "unknown check %s\n", name), 2;
   std::printf("%s: %ld strips, %ld bounded, %d failures\n", name, g_strips, g_bounded, g_failures);
   return g_failures != 0;
