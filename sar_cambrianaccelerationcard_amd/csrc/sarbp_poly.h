@@ -181,31 +181,39 @@ struct PolySetup {
     const float lx = X * sqrtf(uxx), ly = Y * sqrtf(uyy), mu = fabsf(alf) * X / lx;
     const float q1 = lx * invf, q2 = q1 * q1, q4 = q2 * q2;
     const float rad = 6.2831853f * (float)c.k_rev;
+    const float c13 = g3 * (4.0f * bef * (bef * a11 + 2.0f * alf * a02) - 2.0f * a11 * a02);
+    const float c04 = g3 * a02 * (4.0f * bef * bef - a02);
+    const float e13 = X * Y * Y * Y * fabsf(c13) + Y * Y * Y * Y * fabsf(c04);
+    const float l = lx + ly, q = l * invf, ql4 = q * q * q * q;
     if constexpr (PREC == kDF) {
       const float r4 = 4.0f * g2 * g2;
       const float af2 = alf * alf;
       c50 = r4 * alf * a20 * (0.375f * a20 - 0.5f * af2);
       c41 = r4 * (0.375f * a20 * (bef * a20 + 2.0f * alf * a11) - 0.5f * af2 * (alf * a11 + 3.0f * bef * a20));
-      // dropped: y^3 x and y^4, the fifth order's y^2 x^3 (up to 4 (mu + mu^3))
-      // and y^3 x^2, the sixth's x^6 and y x^5
-      const float c13 = g3 * (4.0f * bef * (bef * a11 + 2.0f * alf * a02) - 2.0f * a11 * a02);
+      // Dropped: x y^3 and y^4; the fifth order but for x^5 and x^4 y; the sixth,
+      // along x (mu its cosine) and off it up to ly times the form's largest
+      // gradient, 0.38 |d|^5 / R0^5; and from the seventh on |d| (d / R0)^6 / 16 /
+      // (1 - d / R0).
+      const float bf2 = bef * bef, ab = alf * bef, t22 = 2.0f * a20 * a02 + a11 * a11;
+      const float c32 = r4 * (0.375f * (alf * t22 + 2.0f * bef * a20 * a11) -
+                              0.5f * alf * (af2 * a02 + 3.0f * (ab * a11 + bf2 * a20)));
+      const float c23 = r4 * (0.375f * (2.0f * alf * a11 * a02 + bef * t22) -
+                              0.5f * bef * (3.0f * (af2 * a02 + ab * a11) + bf2 * a20));
+      const float c14 = r4 * (0.375f * a02 * (alf * a02 + 2.0f * bef * a11) - 0.5f * bf2 * (3.0f * alf * a02 + bef * a11));
+      const float c05 = r4 * bef * a02 * (0.375f * a02 - 0.5f * bf2);
+      const float e5 = Y * Y * (X * X * (X * fabsf(c32) + Y * fabsf(c23)) + Y * Y * (X * fabsf(c14) + Y * fabsf(c05)));
       const float mu2 = mu * mu;
-      const float e6 = q1 * (lx * (0.0625f + 0.75f * mu2 + 0.5f * mu2 * mu2) + ly * (0.375f + 1.5f * mu));
-      const float e5 = ly * ly / lx * (4.0f * (mu + mu * mu2) + 0.6f * ly / lx);
-      const float e4 = Y * Y * Y * (X * fabsf(c13) + 4.0f * Y * g3 * bef * bef * a02);
-      mode = bounded && rad * (q4 * (e5 + e6) + e4) <= kCompTol ? 0 : 2;
+      const float e6 = q4 * q1 * lx * (0.0625f + 0.75f * mu2 + 0.5f * mu2 * mu2) + ql4 * q * (0.38f * ly + 0.125f * q * l);
+      mode = bounded && q <= 0.5f && rad * (e13 + e5 + e6) <= kCompTol ? 0 : 2;
     } else {
       // Dropped: x y^3 and y^4 whole; x^2 y^2, x^3 y and y^3 but for their fits;
       // the fifth order, (3 mu - 10 mu^3 + 7 mu^5) / 8 of lx^5 / R0^4 along x
       // (mu its cosine), off it up to ly times the form's largest gradient, 0.42
       // |d|^4 / R0^4; and from the sixth on |d| (d / R0)^5 / 16 / (1 - d / R0).
-      const float c13 = g3 * (4.0f * bef * (bef * a11 + 2.0f * alf * a02) - 2.0f * a11 * a02);
-      const float c04 = g3 * a02 * (4.0f * bef * bef - a02);
-      const float l = lx + ly, q = l * invf, ql4 = q * q * q * q;
       const float e5 = q4 * (0.375f * mu + 1.25f * mu * mu * mu) * lx + ql4 * (0.42f * ly + 0.125f * q * l);
-      const float e4 = Y * Y * (0.5f * X * X * fabsf(c22) + X * Y * fabsf(c13) + Y * Y * fabsf(c04));
+      const float e22 = 0.5f * X * X * Y * Y * fabsf(c22);
       const float e31 = 0.25f * X * X * X * Y * fabsf(c31), e03 = 0.25f * Y * Y * Y * fabsf(c03);
-      const float err1 = rad * (e5 + e4), err0 = err1 + rad * (e31 + e03);
+      const float err1 = rad * (e5 + e22 + e13), err0 = err1 + rad * (e31 + e03);
       mode = !(bounded && q <= 0.5f) ? 2 : (err0 <= kPolyTol[0] ? 0 : (err1 <= kPolyTol[1] ? 1 : 2));
     }
   }

@@ -7,6 +7,7 @@
 //            every pixel's bin with half a bin to spare.
 //   ref      SARBP_PREC_REF: what the accepted mode leaves out stays within its
 //            tolerance, for pixels of any shape (aspect 1:100 to 100:1).
+//   df       the same of SARBP_PREC_DF.
 // Exit status 0 when the named check passes.
 #include <algorithm>
 #include <cmath>
@@ -219,14 +220,14 @@ struct Exact {
   }
 };
 
-double eval(const Poly& p, double x, double y) {
+long double eval(const Poly& p, double x, double y) {
   long double r = 0;
   for (int i = 7; i >= 0; --i) {
     long double t = 0;
     for (int j = 7; j >= 0; --j) t = t * y + p.c[i][j];
     r = r * x + t;
   }
-  return (double)r;
+  return r;
 }
 
 // A strip of PX x PY pixels per lane at range R: pixels of any shape and slant,
@@ -262,51 +263,65 @@ void random_strip(Rng& rng, BpArgs& a, double* tc, double* pos, double lx_max, d
 long g_taken[3];
 double g_worst = 0;
 
-template <int PX, int PY>
-void ref_one(Rng& rng) {
-  BpArgs a;
-  double tc[6], pos[3];
-  random_strip<PX, PY>(rng, a, tc, pos, 512.0, 100.0, 8e5);
-  PolySetup<kSinc8, kRef, PX, PY> ps(a, tc[0], tc[1], tc[2], 0.0, tc, pos);
-  ++g_strips;
-  g_bounded += ps.bounded;
-  ++g_taken[ps.mode];
-  if (ps.mode == 2) return;
-  const Exact ex(a, tc, pos);
-  Poly p = ex.series();
+// The terms that the kernel keeps of a strip's series in a mode.
+template <int PREC, int PX, int PY>
+Poly kept(Poly p, int mode) {
   const double X = 32.0 * PX, Y = 0.5 * (PY - 1);
   for (int i = 0; i < 7; ++i)
     for (int j = 0; i + j < 7; ++j) {
       const long double c = p.c[i][j];
       const int n = i + j;
-      bool keep = n <= 3 || (n == 4 && j <= 1);
-      if (i == 2 && j == 2) p.c[0][2] += 0.5 * X * X * c;
-      if (ps.mode == 0 && i == 3 && j == 1) p.c[1][1] += 0.75 * X * X * c, keep = false;
-      if (ps.mode == 0 && i == 0 && j == 3) p.c[0][1] += 0.75 * Y * Y * c, keep = false;
+      bool keep;
+      if (PREC == kDF) {
+        keep = n <= 3 || (n == 4 && j <= 2) || (n == 5 && j <= 1);
+      } else {
+        keep = n <= 3 || (n == 4 && j <= 1);
+        if (i == 2 && j == 2) p.c[0][2] += 0.5 * X * X * c;
+        if (mode == 0 && i == 3 && j == 1) p.c[1][1] += 0.75 * X * X * c, keep = false;
+        if (mode == 0 && i == 0 && j == 3) p.c[0][1] += 0.75 * Y * Y * c, keep = false;
+      }
       if (!keep) p.c[i][j] = 0;
     }
+  return p;
+}
+
+template <int PREC, int PX, int PY>
+void truncation_one(Rng& rng) {
+  BpArgs a;
+  double tc[6], pos[3];
+  random_strip<PX, PY>(rng, a, tc, pos, PREC == kDF ? 1e5 : 512.0, 100.0, 8e5);
+  PolySetup<kSinc8, PREC, PX, PY> ps(a, tc[0], tc[1], tc[2], 0.0, tc, pos);
+  ++g_strips;
+  g_bounded += ps.bounded;
+  ++g_taken[ps.mode];
+  if (ps.mode == 2) return;
+  const Exact ex(a, tc, pos);
+  const Poly p = kept<PREC, PX, PY>(ex.series(), ps.mode);
+  const double X = 32.0 * PX, Y = 0.5 * (PY - 1), tol = PREC == kDF ? kCompTol : kPolyTol[ps.mode];
   double worst = 0;
   for (int n = 0; n < PY; ++n)
     for (int k = 0; k <= 16; ++k) {
       const double x = -X + k * (2 * X - 1) / 16, y = n - Y;
-      worst = std::max(worst, std::fabs((double)ex.at(x, y) - eval(p, x, y)));
+      worst = std::max(worst, std::fabs((double)(ex.at(x, y) - eval(p, x, y))));
     }
   const double rad = worst * 6.283185307179586 * a.k_rev;
-  g_worst = std::max(g_worst, rad / kPolyTol[ps.mode]);
-  CHECK(rad <= 1.001 * kPolyTol[ps.mode],
-        "PX %d PY %d mode %d: %.3g rad left out, |ux| %.3g |uy| %.3g R %.4g fc %.3g", PX, PY, ps.mode, rad,
-        std::sqrt(tc[3]), std::sqrt(tc[5]), (double)ex.R0, a.k_rev * 1.5e8);
+  g_worst = std::max(g_worst, rad / tol);
+  CHECK(rad <= 1.001 * tol, "PX %d PY %d mode %d: %.3g rad left out, |ux| %.3g |uy| %.3g R %.4g fc %.3g", PX, PY,
+        ps.mode, rad, std::sqrt(tc[3]), std::sqrt(tc[5]), (double)ex.R0, a.k_rev * 1.5e8);
 }
 
-void check_ref() {
+template <int PREC>
+void check_truncation() {
   Rng rng(11);
   for (int i = 0; i < 60000; ++i) {
-    ref_one<1, 2>(rng), ref_one<1, 4>(rng), ref_one<1, 8>(rng);
-    ref_one<2, 2>(rng), ref_one<2, 4>(rng), ref_one<2, 8>(rng);
-    ref_one<4, 2>(rng), ref_one<4, 4>(rng);
+    truncation_one<PREC, 1, 2>(rng), truncation_one<PREC, 1, 4>(rng), truncation_one<PREC, 1, 8>(rng);
+    if constexpr (PREC == kRef) {
+      truncation_one<PREC, 2, 2>(rng), truncation_one<PREC, 2, 4>(rng), truncation_one<PREC, 2, 8>(rng);
+      truncation_one<PREC, 4, 2>(rng), truncation_one<PREC, 4, 4>(rng);
+    }
   }
   // every mode is taken, and the bounds are of the errors' size
-  for (long n : g_taken) CHECK(n > g_strips / 100, "modes taken %ld %ld %ld", g_taken[0], g_taken[1], g_taken[2]);
+  for (int m = 0; m < 3; ++m) CHECK(g_taken[m] > g_strips / 100 || (PREC == kDF && m == 1), "mode %d taken %ld", m, g_taken[m]);
   CHECK(g_worst > 0.5, "largest error %.2f of the tolerance", g_worst);
   std::printf("modes %ld %ld %ld, largest error %.2f of the tolerance\n", g_taken[0], g_taken[1], g_taken[2], g_worst);
 }
@@ -316,7 +331,8 @@ void check_ref() {
 int main(int argc, char** argv) {
   const char* name = argc > 1 ? argv[1] : "";
   if (!std::strcmp(name, "window")) check_window();
-  else if (!std::strcmp(name, "ref")) check_ref();
+  else if (!std::strcmp(name, "ref")) check_truncation<kRef>();
+  else if (!std::strcmp(name, "df")) check_truncation<kDF>();
   else return std::fprintf(stderr, "unknown check %s\n", name), 2;
   std::printf("%s: %ld strips, %ld bounded, %d failures\n", name, g_strips, g_bounded, g_failures);
   return g_failures != 0;

@@ -55,3 +55,12 @@ def _run(precision, interp, ux, uy, rows, R, dr, pulses, axes):
 ])
 def test_long_pixels_match_oracle(interp, ux, uy, rows, R, axes, bound):
     assert _run("ref", interp, ux, uy, rows, R, 0.1875, 48, axes) <= bound
+
+
+# DF: 8e-6 rad left out, FP32 bins up to 500 (a few roundings of 1.8e-5 bin rms)
+@pytest.mark.parametrize("interp,ux,uy,rows,R,dr,axes", [
+    ("sinc8", 0.25, 15.0, 8, 5000.0, 0.75, "xy"), ("linear", 0.25, 25.0, 4, 5000.0, 0.75, "yx"),
+    ("linear", 0.98, 14.5, 8, 8400.0, 0.75, "xy"), ("sinc8", 6.0, 0.1, 4, 5000.0, 0.75, "xy"),
+])
+def test_long_pixels_match_oracle_in_double_float(interp, ux, uy, rows, R, dr, axes):
+    assert _run("df", interp, ux, uy, rows, R, dr, 48, axes) <= 5e-5
