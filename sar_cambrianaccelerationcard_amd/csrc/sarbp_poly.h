@@ -19,6 +19,14 @@ SARBP_HD float float_of_bits(int v) {
   return f;
 }
 
+SARBP_HD float fract_of(float v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_fractf(v);
+#else
+  return v - floorf(v);
+#endif
+}
+
 // 1 / sqrt(v) to 2^-23 or better.
 SARBP_HD double rsqrt_estimate(double v) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -66,21 +74,24 @@ constexpr float kPolyTol[2] = {1.5e-6f, 5e-6f};  // rad, modes 0 and 1
 // first position in the pulse's staged ones.
 //
 // SARBP_PREC_DF takes the same expansion further (x^5, y x^3, y x^4, y^2 x^2,
-// y^3) and evaluates the terms that reach tens of revolutions, pa x + a2 x^2,
-// without rounding: pa and a2 are split into multiples of 2^-17, whose products
-// with the integers x and x^2 and their sum are exact in FP32 and lose their
-// whole revolutions exactly, and FP32 remainders.  The phase is then good to
-// ~4e-7 rad rms (1.5e-6 at most) up to 2 m pixels at 5 km, against 1.4e-6 rms
-// of the double-float form per pixel.  Where the dropped terms exceed
-// kCompTol, or without a bound, every pixel's range and phase are FP64 (mode
-// 2).  1024 x 768 pixels of 1.6 m, 2048 pulses, sinc8: 6.95 ms per pixel in
+// y^3) and evaluates the terms that reach many revolutions, pa x + a2 x^2, without
+// rounding: pa and a2 are split into multiples of 1 / kCompGrid, whose products
+// with the integers x and x^2 and their sum are exact in FP32 up to kCompExact
+// revolutions and lose their whole ones exactly, and FP32 remainders.  The
+// other terms are rounded and may reach kCompTurns revolutions.  The phase is
+// then good to 5e-7 rad rms (1.3e-5 at most, 8e-6 of it left out), against
+// 1.4e-6 rms of the double-float form per pixel.  Where a limit is passed, or
+// without a bound, every pixel's range and phase are FP64 (mode 2).
+// 1024 x 768 pixels of 1.6 m, 2048 pulses, sinc8: 6.95 ms per pixel in
 // double-float, 3.9 by rows.
 // Record: {c0, pa hi, pa lo, a2 hi | a2 lo, A2, A3, A4 | A5, pb, B1, B2 |
 // B3, B4, C0, C1 | C2, D3, bin0, alpha | beta, last bin, -, tag}.  Mode 2:
 // {antenna x, y (FP64) | z, range of the first position (FP64) | .. | -, last
 // bin, -, tag}.
 constexpr float kCompTol = 8e-6f;  // rad, a bound: at it the error is ~1.2e-6 rms
-constexpr double kCompGrid = 131072.0;
+constexpr double kCompGrid = 16384.0;
+constexpr float kCompExact = 1000.0f;  // revolutions: below 2^24 / kCompGrid
+constexpr float kCompTurns = 4.0f;
 
 // Largest bin (the interpolator's unit) of n staged positions or samples.
 template <int INTERP>
@@ -204,7 +215,14 @@ struct PolySetup {
       const float e5 = Y * Y * (X * X * (X * fabsf(c32) + Y * fabsf(c23)) + Y * Y * (X * fabsf(c14) + Y * fabsf(c05)));
       const float mu2 = mu * mu;
       const float e6 = q4 * q1 * lx * (0.0625f + 0.75f * mu2 + 0.5f * mu2 * mu2) + ql4 * q * (0.38f * ly + 0.125f * q * l);
-      mode = bounded && q <= 0.5f && rad * (e13 + e5 + e6) <= kCompTol ? 0 : 2;
+      // Revolutions of the terms that FP32 rounds, and of those it does not.
+      const float kr = (float)c.k_rev, g = 0.5f * invf;
+      const float rounded = X * Y * (g * fabsf(a11) + X * g2 * (fabsf(alf * a11) + fabsf(bef) * a20) +
+                                     Y * g2 * (fabsf(alf) * a02 + fabsf(bef * a11))) +
+                            g * Y * Y * a02 + X * X * X * g2 * fabsf(alf) * a20;
+      const float exact = kr * X * X * g * a20 + 0.5f * X;
+      mode = bounded && q <= 0.5f && rad * (e13 + e5 + e6) <= kCompTol && kr * rounded <= kCompTurns &&
+                     exact <= kCompExact ? 0 : 2;
     } else {
       // Dropped: x y^3 and y^4 whole; x^2 y^2, x^3 y and y^3 but for their fits;
       // the fifth order, (3 mu - 10 mu^3 + 7 mu^5) / 8 of lx^5 / R0^4 along x
@@ -284,6 +302,50 @@ struct PolySetup {
     r[3] = make_float4((float)(c.inv_dr * kS * be) + S * f01, S * c31, (float)c.k_rev * c03, tag);
   }
 };
+
+// The polynomial's terms in y at one column x of the strip: the phase is
+// A + y (B + y^2 D) + y^2 C, the bin b0 + y b1 + y^2 b2.  rk: revolutions per bin
+// unit.
+struct RowTerms {
+  float A, B, C, D, b0, b1, b2;
+};
+
+// Of a SARBP_PREC_REF record, mode 0 or 1.
+template <int MODE>
+SARBP_HD RowTerms ref_row(const float4& p0, const float4& p1, const float4& p2, const float4& p3, float x, float x2,
+                          float rk) {
+#pragma clang fp contract(off)
+  RowTerms t;
+  const float qa = x2 * fmaf(fmaf(p1.x, x, p0.w), x, p0.z);
+  t.A = fmaf(rk, qa, fmaf(p0.y, x, p0.x));
+  t.b0 = fmaf(p2.w, x, p2.z) + qa;
+  const float qb = x * (MODE == 1 ? fmaf(fmaf(p3.y, x, p1.w), x, p1.z) : fmaf(p1.w, x, p1.z));
+  t.B = fmaf(rk, qb, p1.y);
+  t.b1 = p3.x + qb;
+  t.b2 = fmaf(p2.y, x, p2.x);
+  t.C = rk * t.b2;
+  t.D = MODE == 1 ? p3.z : 0.0f;
+  return t;
+}
+
+// Of a SARBP_PREC_DF record, mode 0: the large phase terms exact modulo a
+// revolution.
+SARBP_HD RowTerms comp_row(const float4& p0, const float4& p1, const float4& p2, const float4& p3, const float4& p4,
+                           const float4& p5, float x, float x2, float rk) {
+#pragma clang fp contract(off)
+  RowTerms t;
+  const float turns = fract_of(fmaf(p0.y, x, p0.w * x2));  // exact
+  const float qh = x * fmaf(fmaf(p2.x, x, p1.w), x, p1.z);
+  t.A = turns + fmaf(x2, fmaf(rk, qh, p1.x), fmaf(p0.z, x, p0.x));
+  t.b0 = fmaf(p4.w, x, p4.z) + x2 * (p1.y + qh);
+  const float qb = x * fmaf(fmaf(fmaf(p3.y, x, p3.x), x, p2.w), x, p2.z);
+  t.B = fmaf(rk, qb, p2.y);
+  t.b1 = p5.x + qb;
+  t.b2 = fmaf(fmaf(p4.x, x, p3.w), x, p3.z);
+  t.C = rk * t.b2;
+  t.D = p4.y;
+  return t;
+}
 
 // The setup's constants of one tile: its reference pixel and the grid steps'
 // products (kept in LDS, not in 12 registers through the pixel loop).

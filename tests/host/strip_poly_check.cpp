@@ -8,6 +8,8 @@
 //   ref      SARBP_PREC_REF: what the accepted mode leaves out stays within its
 //            tolerance, for pixels of any shape (aspect 1:100 to 100:1).
 //   df       the same of SARBP_PREC_DF.
+//   df_phase the FP32 phase of accepted SARBP_PREC_DF strips, as the kernel
+//            evaluates it, against the exact one.
 // Exit status 0 when the named check passes.
 #include <algorithm>
 #include <cmath>
@@ -326,6 +328,57 @@ void check_truncation() {
   std::printf("modes %ld %ld %ld, largest error %.2f of the tolerance\n", g_taken[0], g_taken[1], g_taken[2], g_worst);
 }
 
+// Row n's phase (revolutions) and bin from a record's terms, as the pixel loops
+// form them.
+float phase_of(const RowTerms& c, float y) { return fmaf(y, fmaf(y * y, c.D, c.B), fmaf(y * y, c.C, c.A)); }
+float bin_of(const RowTerms& c, float y) { return fmaf(y, c.b1, fmaf(y * y, c.b2, c.b0)); }
+
+double g_sum2 = 0;
+long g_pixels = 0;
+
+template <int PY>
+void df_phase_one(Rng& rng) {
+  BpArgs a;
+  double tc[6], pos[3];
+  random_strip<1, PY>(rng, a, tc, pos, 1e5, 1000.0, 8e5);
+  PolySetup<kSinc8, kDF, 1, PY> ps(a, tc[0], tc[1], tc[2], 0.0, tc, pos);
+  ++g_strips;
+  g_bounded += ps.bounded;
+  ++g_taken[ps.mode];
+  if (ps.mode == 2) return;
+  alignas(16) float4 r[6];
+  ps.store(a, pos, 0, r);
+  const Exact ex(a, tc, pos);
+  const float rk = (float)(a.k_rev * a.dr / bin_scale<kSinc8>());
+  double worst = 0;
+  for (int n = 0; n < PY; ++n)
+    for (int x = -32; x < 32; x += 3) {
+      const float y = n - 0.5f * (PY - 1), xf = (float)x;
+      const float ph = phase_of(comp_row(r[0], r[1], r[2], r[3], r[4], r[5], xf, xf * xf, rk), y);
+      long double e = (long double)a.k_rev * (ex.R0 + ex.at(x, y)) - ph;
+      e -= rintl(e);
+      worst = std::max(worst, (double)fabsl(e) * 6.283185307179586);
+      g_sum2 += (double)(e * e) * 39.4784176;
+      ++g_pixels;
+    }
+  g_worst = std::max(g_worst, worst);
+  // 8e-6 rad left out at most, and sums of up to 8 revolutions rounded a few
+  // times to 2.4e-7 of one
+  CHECK(worst <= 1.3e-5, "PY %d: phase off by %.3g rad, |ux| %.3g |uy| %.3g R %.4g fc %.3g: %.4g revolutions across", PY,
+        worst, std::sqrt(tc[3]), std::sqrt(tc[5]), (double)ex.R0, a.k_rev * 1.5e8,
+        1024 * a.k_rev * (double)(ex.uxx / (2 * ex.R0)));
+}
+
+void check_df_phase() {
+  Rng rng(13);
+  for (int i = 0; i < 60000; ++i) df_phase_one<2>(rng), df_phase_one<4>(rng), df_phase_one<8>(rng);
+  CHECK(g_taken[0] > g_strips / 100 && g_taken[2] > g_strips / 100, "modes %ld %ld", g_taken[0], g_taken[2]);
+  const double rms = std::sqrt(g_sum2 / g_pixels);
+  // the double-float form per pixel: 1.4e-6 rad rms
+  CHECK(rms <= 1.4e-6, "phase error %.3g rad rms", rms);
+  std::printf("modes %ld %ld, phase error %.3g rad rms, %.3g at most\n", g_taken[0], g_taken[2], rms, g_worst);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -333,6 +386,7 @@ int main(int argc, char** argv) {
   if (!std::strcmp(name, "window")) check_window();
   else if (!std::strcmp(name, "ref")) check_truncation<kRef>();
   else if (!std::strcmp(name, "df")) check_truncation<kDF>();
+  else if (!std::strcmp(name, "df_phase")) check_df_phase();
   else return std::fprintf(stderr, "unknown check %s\n", name), 2;
   std::printf("%s: %ld strips, %ld bounded, %d failures\n", name, g_strips, g_bounded, g_failures);
   return g_failures != 0;

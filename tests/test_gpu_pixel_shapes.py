@@ -64,3 +64,13 @@ def test_long_pixels_match_oracle(interp, ux, uy, rows, R, axes, bound):
 ])
 def test_long_pixels_match_oracle_in_double_float(interp, ux, uy, rows, R, dr, axes):
     assert _run("df", interp, ux, uy, rows, R, dr, 48, axes) <= 5e-5
+
+
+# Browse pixels from orbit, hundreds of revolutions across a strip: phase as
+# above (1.4e-6 rad rms), FP32 bins up to 90
+@pytest.mark.parametrize("interp,spacing,rows,R,dr", [
+    ("sinc8", 50.0, 4, 300e3, 15.0), ("linear", 50.0, 8, 300e3, 15.0), ("sinc8", 200.0, 4, 800e3, 60.0),
+    ("linear", 60.0, 2, 800e3, 15.0),
+])
+def test_orbital_pixels_match_oracle_in_double_float(interp, spacing, rows, R, dr):
+    assert _run("df", interp, spacing, spacing, rows, R, dr, 48, "xy") <= 1.2e-5
