@@ -56,16 +56,21 @@ SARBP_HD constexpr double bin_scale() {
 // and third order that are not kept whole are replaced by their best lower-
 // order fit over the strip (x^3 -> 3/4 X^2 x and the like).
 //   mode 0 keeps x^2 .. x^4, y x, y x^2, y^2, y^2 x;
-//   mode 1 adds y x^3 and y^3;
+//   mode 1 adds y x^3 and, in the phase, y^3;
 //   mode 2 evaluates the exact two-step form per pixel, with its bin clamped.
 // The setup takes the first mode whose dropped terms stay below kPolyTol of
-// phase (mode 2 also where the window bound does not hold, as for antennas
-// among the pixels or positions that are not numbers).
+// phase and kBinTol of a bin (mode 2 also where the window bound does not hold,
+// as for antennas among the pixels or positions that are not numbers).  A
+// polynomial's bins are not clamped: that bound and the bin of margin in a
+// strip's positions keep them inside.
 // 4096 x 4096 x 4096 pulses, 0.25 m, sinc8: 59 ms with the expansion per pixel
 // (36.9 VALU instructions and 28.6 issue slots per pixel-pulse, 1 x 4 pixels
 // per lane), 48.3 ms this way at 1 x 8 (27 in the pixel loop), bound by the
 // VALU issue slots at 84% with the LDS pipe 65% busy beside them.
 constexpr float kPolyTol[2] = {1.5e-6f, 5e-6f};  // rad, modes 0 and 1
+// The bin has its own limit, which rules at low carriers and, against the
+// phase's y^3, for rows that are long against dr: its y^3 is the best fit in y.
+constexpr float kBinTol = 4e-6f;  // bins: a tenth of FP32's rounding of bin 500
 // Record of a (pulse, wave), poly_rec16(PREC) float4:
 // {c0, pa, A2, A3 | A4, pb, B1, B2 | C0, C1, bin0, alpha | beta, B3, D3, tag};
 // phases in revolutions, ranges in bin units.  Mode 2: {c0, pa, 2 R0, last bin
@@ -221,8 +226,9 @@ struct PolySetup {
                                      Y * g2 * (fabsf(alf) * a02 + fabsf(bef * a11))) +
                             g * Y * Y * a02 + X * X * X * g2 * fabsf(alf) * a20;
       const float exact = kr * X * X * g * a20 + 0.5f * X;
-      mode = bounded && q <= 0.5f && rad * (e13 + e5 + e6) <= kCompTol && kr * rounded <= kCompTurns &&
-                     exact <= kCompExact ? 0 : 2;
+      const float err = e13 + e5 + e6, e03 = 0.25f * Y * Y * Y * fabsf(c03);
+      mode = bounded && q <= 0.5f && rad * err <= kCompTol && inv_drf * (err + e03) <= kBinTol &&
+                     kr * rounded <= kCompTurns && exact <= kCompExact ? 0 : 2;
     } else {
       // Dropped: x y^3 and y^4 whole; x^2 y^2, x^3 y and y^3 but for their fits;
       // the fifth order, (3 mu - 10 mu^3 + 7 mu^5) / 8 of lx^5 / R0^4 along x
@@ -231,8 +237,10 @@ struct PolySetup {
       const float e5 = q4 * (0.375f * mu + 1.25f * mu * mu * mu) * lx + ql4 * (0.42f * ly + 0.125f * q * l);
       const float e22 = 0.5f * X * X * Y * Y * fabsf(c22);
       const float e31 = 0.25f * X * X * X * Y * fabsf(c31), e03 = 0.25f * Y * Y * Y * fabsf(c03);
-      const float err1 = rad * (e5 + e22 + e13), err0 = err1 + rad * (e31 + e03);
-      mode = !(bounded && q <= 0.5f) ? 2 : (err0 <= kPolyTol[0] ? 0 : (err1 <= kPolyTol[1] ? 1 : 2));
+      const float err1 = e5 + e22 + e13, err0 = err1 + e31 + e03;
+      const bool mode0 = rad * err0 <= kPolyTol[0] && inv_drf * err0 <= kBinTol;
+      const bool mode1 = rad * err1 <= kPolyTol[1] && inv_drf * (err1 + e03) <= kBinTol;
+      mode = !(bounded && q <= 0.5f) ? 2 : (mode0 ? 0 : (mode1 ? 1 : 2));
     }
   }
 
@@ -265,7 +273,7 @@ struct PolySetup {
     c0 -= floor(c0);
     const float b0 = (float)(kS * (bin0 - (double)first));
     const float tag = float_of_bits((offset << 2) | mode);
-    const float g = (float)(0.5 * inv);
+    const float g = (float)(0.5 * inv), f01 = 0.75f * Y * Y * c03;
     if constexpr (PREC == kDF) {
       if (mode == 2) {
         double* d = reinterpret_cast<double*>(r);
@@ -282,7 +290,7 @@ struct PolySetup {
       r[2] = make_float4(S * c50, (float)pb, S * g * a11, -S * g2 * (alf * a11 + bef * a20));
       r[3] = make_float4(S * c31, S * c41, S * g * a02, -S * g2 * (alf * a02 + bef * a11));
       r[4] = make_float4(S * c22, (float)c.k_rev * c03, b0, (float)(c.inv_dr * kS * al));
-      r[5] = make_float4((float)(c.inv_dr * kS * be), (float)bin_last<INTERP>(n), 0.0f, tag);
+      r[5] = make_float4((float)(c.inv_dr * kS * be) + S * f01, (float)bin_last<INTERP>(n), 0.0f, tag);
       return;
     }
     if (mode == 2) {
@@ -292,10 +300,10 @@ struct PolySetup {
       r[3] = make_float4(bef, 0.0f, 0.0f, tag);
       return;
     }
-    // mode 0: x^3 y and y^3 as their best fits in x y and y
-    const float f11 = mode == 0 ? 0.75f * X * X * c31 : 0.0f, f01 = mode == 0 ? 0.75f * Y * Y * c03 : 0.0f;
+    // mode 0: x^3 y and, in the phase too, y^3 as their best fits in x y and y
+    const float f11 = mode == 0 ? 0.75f * X * X * c31 : 0.0f;
     r[0] = make_float4((float)c0, (float)pa, (float)(c.inv_dr * kS * c20), -S * g2 * alf * a20);
-    r[1] = make_float4(S * g3 * a20 * (4.0f * alf * alf - a20), (float)pb + (float)c.k_rev * f01,
+    r[1] = make_float4(S * g3 * a20 * (4.0f * alf * alf - a20), (float)pb + (mode == 0 ? (float)c.k_rev * f01 : 0.0f),
                        S * (g * a11 + f11), -S * g2 * (alf * a11 + bef * a20));
     r[2] = make_float4(S * (g * a02 + 0.5f * X * X * c22), -S * g2 * (alf * a02 + bef * a11), b0,
                        (float)(c.inv_dr * kS * al));

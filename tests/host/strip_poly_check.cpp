@@ -10,6 +10,8 @@
 //   df       the same of SARBP_PREC_DF.
 //   df_phase the FP32 phase of accepted SARBP_PREC_DF strips, as the kernel
 //            evaluates it, against the exact one.
+//   bins     the same of the bins, of REF and DF, at any carrier down to none:
+//            within FP32 rounding of the exact ones and inside the positions.
 // Exit status 0 when the named check passes.
 #include <algorithm>
 #include <cmath>
@@ -379,6 +381,59 @@ void check_df_phase() {
   std::printf("modes %ld %ld, phase error %.3g rad rms, %.3g at most\n", g_taken[0], g_taken[2], rms, g_worst);
 }
 
+template <int INTERP, int PREC, int PX, int PY>
+void bins_one(Rng& rng) {
+  BpArgs a;
+  double tc[6], pos[3];
+  random_strip<PX, PY>(rng, a, tc, pos, PREC == kDF ? 1e5 : 512.0, 100.0, 8e5);
+  a.k_rev *= std::pow(10.0, -(int)(rng() % 8));
+  if (rng() % 8 == 0) a.k_rev = 0;
+  PolySetup<INTERP, PREC, PX, PY> ps(a, tc[0], tc[1], tc[2], 0.0, tc, pos);
+  ++g_strips;
+  g_bounded += ps.bounded;
+  ++g_taken[ps.mode];
+  if (ps.mode == 2) return;
+  alignas(16) float4 r[6];
+  ps.store(a, pos, 0, r);
+  const Exact ex(a, tc, pos);
+  const double scale = bin_scale<INTERP>() * a.inv_dr, first = bin_scale<INTERP>() * (ps.first * a.dr + a.r0 - (double)ex.R0) * a.inv_dr;
+  const float rk = (float)(a.k_rev * a.dr / bin_scale<INTERP>());
+  double worst = 0, largest = 0;
+  for (int n = 0; n < PY; ++n)
+    for (int x = -32 * PX; x < 32 * PX; x += 5) {
+      const float y = n - 0.5f * (PY - 1), xf = (float)x;
+      RowTerms t;
+      if constexpr (PREC == kDF)
+        t = comp_row(r[0], r[1], r[2], r[3], r[4], r[5], xf, xf * xf, rk);
+      else
+        t = ps.mode == 1 ? ref_row<1>(r[0], r[1], r[2], r[3], xf, xf * xf, rk)
+                         : ref_row<0>(r[0], r[1], r[2], r[3], xf, xf * xf, rk);
+      const float bin = bin_of(t, y);
+      const double exact = (double)(ex.at(x, y) * scale - first);
+      worst = std::max(worst, std::fabs(bin - exact));
+      largest = std::max(largest, exact);
+      CHECK(bin >= 0.0f && bin < (float)bin_last<INTERP>(ps.n) + (INTERP == kLinear ? 0.0f : 1.0f),
+            "bin %g outside the %d positions", bin, ps.n);
+    }
+  // what is left out (kBinTol bins, at the interpolator's scale) and six
+  // roundings of the largest
+  const double allowed = bin_scale<INTERP>() * kBinTol + 6 * std::ldexp(largest, -24);
+  g_worst = std::max(g_worst, worst / allowed);
+  CHECK(worst <= allowed, "PREC %d PX %d PY %d mode %d: bin off by %.3g of %.4g, |ux| %.3g |uy| %.3g R %.4g fc %.3g dr %.3g", PREC, PX,
+        PY, ps.mode, worst, largest, std::sqrt(tc[3]), std::sqrt(tc[5]), (double)ex.R0, a.k_rev * 1.5e8, a.dr);
+}
+
+void check_bins() {
+  Rng rng(17);
+  for (int i = 0; i < 30000; ++i) {
+    bins_one<kLinear, kRef, 1, 2>(rng), bins_one<kSinc8, kRef, 1, 4>(rng), bins_one<kSinc8W, kRef, 1, 8>(rng);
+    bins_one<kSinc8, kRef, 2, 8>(rng), bins_one<kLinear, kRef, 4, 4>(rng), bins_one<kSinc8, kDF, 1, 2>(rng);
+    bins_one<kLinear, kDF, 1, 4>(rng), bins_one<kSinc8W, kDF, 1, 8>(rng);
+  }
+  for (long n : g_taken) CHECK(n > g_strips / 200, "modes taken %ld %ld %ld", g_taken[0], g_taken[1], g_taken[2]);
+  std::printf("modes %ld %ld %ld, largest error %.2f of the allowed\n", g_taken[0], g_taken[1], g_taken[2], g_worst);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -387,6 +442,7 @@ int main(int argc, char** argv) {
   else if (!std::strcmp(name, "ref")) check_truncation<kRef>();
   else if (!std::strcmp(name, "df")) check_truncation<kDF>();
   else if (!std::strcmp(name, "df_phase")) check_df_phase();
+  else if (!std::strcmp(name, "bins")) check_bins();
   else return std::fprintf(stderr, "unknown check %s\n", name), 2;
   std::printf("%s: %ld strips, %ld bounded, %d failures\n", name, g_strips, g_bounded, g_failures);
   return g_failures != 0;
