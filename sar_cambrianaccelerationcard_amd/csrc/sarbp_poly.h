@@ -74,9 +74,12 @@ constexpr float kBinTol = 4e-6f;  // bins: a tenth of FP32's rounding of bin 500
 // Record of a (pulse, wave), poly_rec16(PREC) float4:
 // {c0, pa, A2, A3 | A4, pb, B1, B2 | C0, C1, bin0, alpha | beta, B3, D3, tag};
 // phases in revolutions, ranges in bin units.  Mode 2: {c0, pa, 2 R0, last bin
-// | g, pb, 2 g^2, - | -, -, bin0, alpha | beta, -, -, tag} with alpha and beta
-// in m.  tag: the mode in bits 0-1, above them the byte offset of the strip's
-// first position in the pulse's staged ones.
+// | g, pb, 2 g^2, - | first bin, -, bin0, alpha | beta, -, -, tag} with alpha and
+// beta in m.  tag: the mode in bits 0-1, above them the byte offset of the
+// position that the strip's bins count from, in the pulse's staged ones: the
+// one below the centre's bin, so that FP32 rounds the bins at half their span
+// (from the first position on, 1 m pixels with columns along range were up to
+// 1.3 times further from the exact image than the double-float form).
 //
 // SARBP_PREC_DF takes the same expansion further (x^5, y x^3, y x^4, y^2 x^2,
 // y^3) and evaluates the terms that reach many revolutions, pa x + a2 x^2, without
@@ -90,8 +93,8 @@ constexpr float kBinTol = 4e-6f;  // bins: a tenth of FP32's rounding of bin 500
 // 1024 x 768 pixels of 1.6 m, 2048 pulses, sinc8: 6.95 ms per pixel in
 // double-float, 3.9 by rows.
 // Record: {c0, pa hi, pa lo, a2 hi | a2 lo, A2, A3, A4 | A5, pb, B1, B2 |
-// B3, B4, C0, C1 | C2, D3, bin0, alpha | beta, last bin, -, tag}.  Mode 2:
-// {antenna x, y (FP64) | z, range of the first position (FP64) | .. | -, last
+// B3, B4, C0, C1 | C2, D3, bin0, alpha | beta, -, -, tag}.  Mode 2: {antenna x, y
+// (FP64) | z, range of the counted-from position (FP64) | .. | first bin, last
 // bin, -, tag}.
 constexpr float kCompTol = 8e-6f;  // rad, a bound: at it the error is ~1.2e-6 rms
 constexpr double kCompGrid = 16384.0;
@@ -255,7 +258,7 @@ struct PolySetup {
   }
 
   // The record of a strip whose positions begin `offset` bytes into the
-  // pulse's staged ones; bins count from `first`.
+  // pulse's staged ones.
   SARBP_HD void store(const BpArgs& a, const double* pos, int offset, float4* r) const {
 #pragma clang fp contract(off)
     const SetupArgs c(a);
@@ -271,15 +274,17 @@ struct PolySetup {
     pb -= turns;
     double c0 = fma(c.k_rev, R0, -turns * (0.5 * (PY - 1)));
     c0 -= floor(c0);
-    const float b0 = (float)(kS * (bin0 - (double)first));
-    const float tag = float_of_bits((offset << 2) | mode);
+    const int base = bounded ? (int)floor(bin0) - first : 0;
+    const float b0 = (float)(kS * (bin0 - (double)(first + base)));
+    const float lowest = (float)(-kS * base), highest = (float)(bin_last<INTERP>(n) - kS * base);
+    const float tag = float_of_bits(((offset + base * room_bytes(INTERP)) << 2) | mode);
     const float g = (float)(0.5 * inv), f01 = 0.75f * Y * Y * c03;
     if constexpr (PREC == kDF) {
       if (mode == 2) {
         double* d = reinterpret_cast<double*>(r);
         for (int k = 0; k < 3; ++k) d[k] = pos[k];
-        d[3] = fma((double)first, a.dr, c.r0);
-        r[5] = make_float4(0.0f, (float)bin_last<INTERP>(n), 0.0f, tag);
+        d[3] = fma((double)(first + base), a.dr, c.r0);
+        r[5] = make_float4(lowest, highest, 0.0f, tag);
         return;
       }
       const double a2 = c.k_rev * c20;
@@ -290,13 +295,13 @@ struct PolySetup {
       r[2] = make_float4(S * c50, (float)pb, S * g * a11, -S * g2 * (alf * a11 + bef * a20));
       r[3] = make_float4(S * c31, S * c41, S * g * a02, -S * g2 * (alf * a02 + bef * a11));
       r[4] = make_float4(S * c22, (float)c.k_rev * c03, b0, (float)(c.inv_dr * kS * al));
-      r[5] = make_float4((float)(c.inv_dr * kS * be) + S * f01, (float)bin_last<INTERP>(n), 0.0f, tag);
+      r[5] = make_float4((float)(c.inv_dr * kS * be) + S * f01, 0.0f, 0.0f, tag);
       return;
     }
     if (mode == 2) {
-      r[0] = make_float4((float)c0, (float)pa, (float)(2.0 * R0), (float)bin_last<INTERP>(n));
+      r[0] = make_float4((float)c0, (float)pa, (float)(2.0 * R0), highest);
       r[1] = make_float4(g, (float)pb, g2, 0.0f);
-      r[2] = make_float4(0.0f, 0.0f, b0, alf);
+      r[2] = make_float4(lowest, 0.0f, b0, alf);
       r[3] = make_float4(bef, 0.0f, 0.0f, tag);
       return;
     }

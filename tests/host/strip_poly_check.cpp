@@ -11,7 +11,8 @@
 //   df_phase the FP32 phase of accepted SARBP_PREC_DF strips, as the kernel
 //            evaluates it, against the exact one.
 //   bins     the same of the bins, of REF and DF, at any carrier down to none:
-//            within FP32 rounding of the exact ones and inside the positions.
+//            within FP32 rounding (at their distance from the centre's) of the
+//            exact ones and inside the positions.
 // Exit status 0 when the named check passes.
 #include <algorithm>
 #include <cmath>
@@ -396,7 +397,11 @@ void bins_one(Rng& rng) {
   alignas(16) float4 r[6];
   ps.store(a, pos, 0, r);
   const Exact ex(a, tc, pos);
-  const double scale = bin_scale<INTERP>() * a.inv_dr, first = bin_scale<INTERP>() * (ps.first * a.dr + a.r0 - (double)ex.R0) * a.inv_dr;
+  int tag;
+  std::memcpy(&tag, &r[poly_rec16(PREC) - 1].w, 4);
+  const int base = (tag >> 2) / room_bytes(INTERP);  // the position the bins count from
+  const double scale = bin_scale<INTERP>() * a.inv_dr;
+  const double first = bin_scale<INTERP>() * ((ps.first + base) * a.dr + a.r0 - (double)ex.R0) * a.inv_dr;
   const float rk = (float)(a.k_rev * a.dr / bin_scale<INTERP>());
   double worst = 0, largest = 0;
   for (int n = 0; n < PY; ++n)
@@ -411,13 +416,14 @@ void bins_one(Rng& rng) {
       const float bin = bin_of(t, y);
       const double exact = (double)(ex.at(x, y) * scale - first);
       worst = std::max(worst, std::fabs(bin - exact));
-      largest = std::max(largest, exact);
-      CHECK(bin >= 0.0f && bin < (float)bin_last<INTERP>(ps.n) + (INTERP == kLinear ? 0.0f : 1.0f),
-            "bin %g outside the %d positions", bin, ps.n);
+      largest = std::max(largest, std::fabs(exact + first));
+      const double at = bin + bin_scale<INTERP>() * base;
+      CHECK(at >= 0 && at < bin_last<INTERP>(ps.n) + (INTERP == kLinear ? 0 : 1), "bin %g outside the %d positions",
+            at, ps.n);
     }
   // what is left out (kBinTol bins, at the interpolator's scale) and six
-  // roundings of the largest
-  const double allowed = bin_scale<INTERP>() * kBinTol + 6 * std::ldexp(largest, -24);
+  // roundings of the largest distance from the centre's bin
+  const double allowed = bin_scale<INTERP>() * kBinTol + 6 * std::ldexp(largest + 1, -24);
   g_worst = std::max(g_worst, worst / allowed);
   CHECK(worst <= allowed, "PREC %d PX %d PY %d mode %d: bin off by %.3g of %.4g, |ux| %.3g |uy| %.3g R %.4g fc %.3g dr %.3g", PREC, PX,
         PY, ps.mode, worst, largest, std::sqrt(tc[3]), std::sqrt(tc[5]), (double)ex.R0, a.k_rev * 1.5e8, a.dr);
