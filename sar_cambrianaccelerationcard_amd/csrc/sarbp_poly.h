@@ -36,6 +36,22 @@ SARBP_HD double rsqrt_estimate(double v) {
 #endif
 }
 
+// 1 / v and sqrt(v) to an ulp, for bounds.
+SARBP_HD float rcp_estimate(float v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_rcpf(v);
+#else
+  return 1.0f / v;
+#endif
+}
+SARBP_HD float sqrt_estimate(float v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_sqrtf(v);
+#else
+  return sqrtf(v);
+#endif
+}
+
 template <int INTERP>
 SARBP_HD constexpr double bin_scale() {
   return INTERP == kSinc8 ? 2.0 : 1.0;
@@ -166,7 +182,7 @@ struct PolySetup {
     const float smin = fminf(-alf * X, alf * (X - 1.0f)) - fabsf(bef) * Y;
     const float smax = fmaxf(-alf * X, alf * (X - 1.0f)) + fabsf(bef) * Y;
     const float r0f = (float)R0, xlo = r0f + smin, dmax = (float)c.dmax;
-    const float up = smax + dmax * dmax / (2.0f * xlo);
+    const float up = smax + 0.5f * dmax * dmax * rcp_estimate(xlo);
     const double ulo = fma((double)smin, c.inv_dr, bin0);
     const double uhi = fma((double)up, c.inv_dr, bin0);
     // The strip's positions have to lie inside the window that whole_window
@@ -178,7 +194,7 @@ struct PolySetup {
     constexpr int kOff = sinc_rows(INTERP) > 0 ? 3 : 0, kEnd = sinc_rows(INTERP) > 0 ? 2 : 3;
     const float ycf = (float)yc, inv_drf = (float)c.inv_dr;
     const float m = fmaf(ycf * ycf, (float)tc[5], -2.0f * ycf * bef * r0f);
-    const float ref = m / (r0f + sqrtf(fmaf(r0f, r0f, m)));
+    const float ref = m * rcp_estimate(r0f + sqrt_estimate(fmaf(r0f, r0f, m)));
     const bool inside = (smin - ref) * inv_drf >= (float)(kOff + 2 - c.half) + 0.1f &&
                         (up - ref) * inv_drf <= (float)(kOff + window_room(INTERP, c.win) - c.half - kEnd - 1) - 0.1f;
     bounded = inside && xlo > 0.5f * r0f && fabs(ulo) < 1.0e9 && fabs(uhi) < 1.0e9;
@@ -197,7 +213,7 @@ struct PolySetup {
     c31 = g3 * (4.0f * alf * (alf * a11 + 2.0f * bef * a20) - 2.0f * a20 * a11);
     c22 = g3 * (4.0f * (alf * alf * a02 + bef * (2.0f * alf * a11 + bef * a20)) - 2.0f * a20 * a02 - a11 * a11);
     c03 = -g2 * bef * a02;
-    const float lx = X * sqrtf(uxx), ly = Y * sqrtf(uyy), mu = fabsf(alf) * X / lx;
+    const float lx = X * sqrt_estimate(uxx), ly = Y * sqrt_estimate(uyy), mu = fabsf(alf) * X * rcp_estimate(lx);
     const float q1 = lx * invf, q2 = q1 * q1, q4 = q2 * q2;
     const float rad = 6.2831853f * (float)c.k_rev;
     const float c13 = g3 * (4.0f * bef * (bef * a11 + 2.0f * alf * a02) - 2.0f * a11 * a02);
