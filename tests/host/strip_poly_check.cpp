@@ -13,6 +13,7 @@
 //   bins     the same of the bins, of REF and DF, at any carrier down to none:
 //            within FP32 rounding (at their distance from the centre's) of the
 //            exact ones and inside the positions.
+//   root     the FP64 square root of the per-pixel fallback: two roundings.
 // Exit status 0 when the named check passes.
 #include <algorithm>
 #include <cmath>
@@ -440,6 +441,19 @@ void check_bins() {
   std::printf("modes %ld %ld %ld, largest error %.2f of the allowed\n", g_taken[0], g_taken[1], g_taken[2], g_worst);
 }
 
+void check_root() {
+  Rng rng(19);
+  double worst = 0;
+  for (int i = 0; i < 1000000; ++i) {
+    const double r = log_uniform(rng, 1e-3, 1e8), v = r * r;
+    const long double exact = sqrtl((long double)v);
+    worst = std::max(worst, (double)(fabsl(range_root(v) - exact) / exact));
+  }
+  CHECK(worst <= std::ldexp(1.0, -52), "root off by 2^%.2f", std::log2(worst));
+  CHECK(range_root(0.0) == 0.0, "root of 0 is %g", range_root(0.0));
+  std::printf("largest error 2^%.2f\n", std::log2(worst));
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -449,6 +463,7 @@ int main(int argc, char** argv) {
   else if (!std::strcmp(name, "df")) check_truncation<kDF>();
   else if (!std::strcmp(name, "df_phase")) check_df_phase();
   else if (!std::strcmp(name, "bins")) check_bins();
+  else if (!std::strcmp(name, "root")) check_root();
   else return std::fprintf(stderr, "unknown check %s\n", name), 2;
   std::printf("%s: %ld strips, %ld bounded, %d failures\n", name, g_strips, g_bounded, g_failures);
   return g_failures != 0;
