@@ -71,6 +71,7 @@ struct BpArgs {
   int32_t pool;           // row polynomials: staged positions (samples) the LDS holds, else 0
   int32_t parts;          // waves that share a strip's pulses out (1: one workgroup per tile)
   int32_t sum_pulses;     // pulses per partial sum of a pixel (>= 1)
+  float split_limit;      // > 0: the kernels share pulses out only where split_cost stays below it
   int32_t kernel_interp;  // kNearest, kLinear, kSinc8 or kSinc8W
   int32_t kernel_prec;    // kRef, kF64, kF32 or kDF: the arithmetic launched
   // tap-polynomial rows of 4 (sinc8_kernel_rows): kSinc8 [6][P, Q] of the
@@ -112,6 +113,9 @@ __host__ __device__ inline int poly_batch(int P, int rec16) {
   return rec16 > 4 ? n / 2 : n;
 }
 constexpr int kMaxParts = 8;  // waves a split strip's pulses are shared out to
+// LDS of one such wave's staged positions: 8 waves take 62 KB, two workgroups
+// share a CU.
+constexpr int kSplitStage = 5632;
 
 // LDS layout of one workgroup (byte offsets), SB = setup_batch(P):
 //   raw   [P][win] float2         staged range windows (nearest, linear)

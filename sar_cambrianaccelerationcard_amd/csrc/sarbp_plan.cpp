@@ -6,6 +6,7 @@
 // batch grouping.  Nothing here exits or throws.
 #include "sarbp.h"
 #include "sarbp_host.h"
+#include "sarbp_poly.h"
 
 #include <algorithm>
 #include <atomic>
@@ -522,34 +523,43 @@ size_t launch_lds(const BpArgs& a) {
 // planned window, so a smaller pool still holds several: 3584^2 x 1024 pulses
 // at 1 m (324-sample windows) ran 31.8 ms with 56 KB of LDS, 23.9 ms with 40;
 // 2560^2 at 0.5 m (104 samples) 7.4 ms with 42.5 KB, 6.7 ms with 40.
-int stage_pool(int kinterp, int kprec, int win, int P, int most) {
+// An image with fewer tiles than fill the CUs four deep shares them out to
+// fewer: 1 m, columns along range, sinc8, 1024 pulses, one and two tiles per CU
+// 2143 -> 1693 and 2221 -> 1755 us, three 2601 -> 2187; 0.25 m across 498 -> 494.
+int stage_pool(int kinterp, int kprec, int win, int P, int most, int64_t tiles) {
   const int room = window_room(kinterp, win), bytes = room_bytes(kinterp);
   const size_t fixed = lds_layout(kinterp, win, P, 16, poly_rec16(kprec)).total - 16 * (size_t)bytes;
-  for (int per_cu = 4; per_cu > 1; --per_cu) {
+  const int deep = (int)std::max<int64_t>(2, std::min<int64_t>(4, (tiles + 255) / 256));
+  // such an image's stage is as deep as the LDS allows
+  if (deep < 4) most = poly_batch(P, poly_rec16(kprec));
+  for (int per_cu = deep; per_cu > 1; --per_cu) {
     const size_t budget = std::min(kLdsBudget, (kCuLds / per_cu - kBatchStaticLds) & ~(size_t)255);
     if (fixed + (size_t)room * bytes <= budget) return (int)std::min<size_t>((size_t)most * room, (budget - fixed) / bytes);
   }
-  return most * room;
+  return room;
 }
 
-// Partial sums that a job's pulses are split into, a wave of its strip each:
-// as many as keep the waves within four rounds of the 4096 that the chip
-// holds (256 CUs x 16), with 16 pulses or more in each.  1024 pulses, unsplit
-// against split: 96^2 475 -> 83 us, 512^2 499 -> 281, 768^2 801 -> 630 (sinc8,
-// 0.25 m), 512^2 355 -> 177, 1024^2 727 -> 660 (linear).  A sinc8 strip makes
-// the coefficients of its positions (`room` at most) alone, where a workgroup
-// per tile shares them among four: from 2560 strips or 2^19 positions a pulse
-// on that costs more than the split gains.  Unsplit against split, us, at
-// strips x room: 0.25 m 4096 x 65 1041 / 1058; 0.7 m 2304 x 101 1101 / 905,
-// 3072 x 109 1245 / 1344; 1.25 m 2304 x 213 1603 / 1438, 3072 x 237 1727 /
-// 2432; 1.6 m 1024 x 261 1285 / 887, 2304 x 301 1763 / 2219; 2 m 2304 x 417
-// 2032 / 2847.
-int pulse_parts(int kinterp, int64_t strips, int room, int n_pulses) {
-  constexpr int64_t kWaveRounds = 4 * 4096, kSinc8Strips = 2560, kSinc8Positions = 1 << 19;
-  if (kinterp != kLinear && (strips > kSinc8Strips || strips * room > kSinc8Positions)) return 1;
+// Partial sums that a job's pulses may be split into, a wave of its strip each:
+// as many as keep the waves within four rounds of the 4096 that the chip holds
+// (256 CUs x 16), with 16 pulses or more in each.
+int pulse_parts(int64_t strips, int n_pulses) {
   int parts = 1;
-  while (parts < kMaxParts && strips * parts * 2 <= kWaveRounds && n_pulses >= 32 * parts) parts *= 2;
+  while (parts < kMaxParts && strips * parts * 2 <= 4 * 4096 && n_pulses >= 32 * parts) parts *= 2;
   return parts;
+}
+
+// The split_cost from which splitting does not pay: one over the share of its
+// full rate that the chip reaches on an image of so many strips, a workgroup
+// per tile (measured 0.11 / 0.28 / 0.43 / 0.56 / 0.67 / 0.86 / 0.95 at 256 / 576 /
+// 1024 / 1536 / 2304 / 3072 / 4096, at every spacing and orientation; where few
+// tiles have room for deep stages, up to a fifth more).  1024 pulses, sinc8,
+// unsplit against split: 0.25 m columns across range 512^2 498 -> 259 us, 768^2
+// 769 -> 529; 0.5 m along it, split_cost 3.3, 256^2 1026 -> 438, 512^2 918 and
+// 1214, 768^2 1361 and 2794.  Linear, 0.5 m: across 1024 x 768 526 -> 424, along
+// 675 and 901; its split strips pay up to twice as many.
+double split_limit(int kinterp, int64_t strips) {
+  if (strips > 4096 && kinterp != kLinear) return 0.0;
+  return 1.0 / (strips <= 1024 ? 0.05 + strips / 2400.0 : std::min(1.0, 0.477 + (strips - 1024) / 5870.0));
 }
 
 // Fills a launch descriptor.  Caller holds ctx->mu and the device guard.
@@ -629,12 +639,23 @@ sarbp_status plan_args(const double* h_pos, const sarbp_grid* g,
   a->parts = 1;
   a->sum_pulses = INT32_MAX;
   if (row_polynomials(kinterp, kprec)) {
-    a->pool = stage_pool(kinterp, kprec, win, P, plain);
-    if (px == 1) {
-      a->parts = pulse_parts(kinterp, (int64_t)a->tiles_x * a->tiles_y * kWaves, window_room(kinterp, win),
-                             p->n_pulses);
-      if (a->parts > 1) a->sum_pulses = (p->n_pulses + a->parts - 1) / a->parts;
+    const int64_t tiles = (int64_t)a->tiles_x * a->tiles_y;
+    // a batch's launch is shared with other jobs
+    a->pool = stage_pool(kinterp, kprec, win, P, plain, batched ? INT32_MAX : tiles);
+    int parts = px == 1 ? pulse_parts(tiles * kWaves, p->n_pulses) : 1;
+    if (parts > 1) {
+      const float limit = (float)split_limit(kinterp, tiles * kWaves);
+      const float along = touched(norm3(g->ux), 0.0, py, a->inv_dr);
+      if (limit == 0.0f || (h_pos && !split_wins(*a, h_pos, py, limit))) {
+        parts = 1;
+      } else if (!h_pos && split_cost(kinterp, kprec, py, along, along) >= limit) {
+        // columns along range would not split: without the positions the
+        // kernels look
+        a->split_limit = limit;
+      }
     }
+    a->parts = parts;
+    if (parts > 1) a->sum_pulses = (p->n_pulses + parts - 1) / parts;
   }
   sinc8_kernel_rows(kinterp, p->kaiser_beta, a->sinc_poly);
   if (info) {

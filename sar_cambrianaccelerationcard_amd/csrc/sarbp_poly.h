@@ -387,6 +387,49 @@ SARBP_HD RowTerms comp_row(const float4& p0, const float4& p1, const float4& p2,
   return t;
 }
 
+// A strip-pulse's work where its own wave stages its positions, over its work
+// where a workgroup stages the tile's for four: `strip` and `tile` are the
+// positions (samples) touched.  In units of a staged position, a row of 64
+// pixels costs 6.25 (sinc8) or 37 (linear), again for every piece that the
+// strip's positions are staged in.  Fitted to the throughput of 2048^2 images
+// against split 768^2 and 1024^2 ones, columns across, along and at 45 degrees
+// to range at 0.25 to 1.6 m: within 25% of the measured ratios of 0.9 to 3.3.
+SARBP_HD float split_cost(int interp, int prec, int rows, float strip, float tile) {
+  const bool sinc = sinc_rows(interp) > 0;
+  const float pixels = (sinc ? 6.25f : 37.0f) * (float)rows;
+  const float pieces = ceilf(strip / (float)(kSplitStage / room_bytes(interp)));
+  const float scale = (sinc ? 1.0f : 0.88f) * (prec == kDF ? 1.1f : 1.0f);
+  return scale * (pixels * fmaxf(pieces, 1.0f) + strip) / (pixels + 0.25f * tile);
+}
+// Positions that a strip of 64 columns by `rows` rows touches, of range steps dx
+// and dy (m) a pixel.
+SARBP_HD float touched(double dx, double dy, int rows, double inv_dr) {
+  return (float)((dx * (kTileX - 1) + dy * (rows - 1)) * inv_dr) + 3.5f;
+}
+
+// Whether a job's strips cost less than `limit` split, by the mean range steps at
+// two quarter points of the image from the first, the middle and the last of
+// its antenna positions.  A position that is no number does not split.
+SARBP_HD bool split_wins(const BpArgs& a, const double* pos, int rows, float limit) {
+  double dx = 0.0, dy = 0.0;
+  for (int m = 0; m < 6; ++m) {
+    const double* p = pos + 3 * (size_t)(m % 3 == 0 ? 0 : (m % 3 == 1 ? a.n_pulses / 2 : a.n_pulses - 1));
+    const double at = m < 3 ? 0.25 : 0.75;
+    double r2 = 0.0, al = 0.0, be = 0.0;
+    for (int k = 0; k < 3; ++k) {
+      const double e = a.origin[k] + at * a.nx * a.ux[k] + at * a.ny * a.uy[k] - p[k];
+      r2 += e * e;
+      al += e * a.ux[k];
+      be += e * a.uy[k];
+    }
+    const double sixth = (1.0 / 6.0) * rsqrt_estimate(r2);
+    dx += fabs(al) * sixth;
+    dy += fabs(be) * sixth;
+  }
+  return split_cost(a.kernel_interp, a.kernel_prec, rows, touched(dx, dy, rows, a.inv_dr),
+                    touched(dx, dy, kWaves * rows, a.inv_dr)) < limit;
+}
+
 // The setup's constants of one tile: its reference pixel and the grid steps'
 // products (kept in LDS, not in 12 registers through the pixel loop).
 SARBP_HD void tile_constants(const BpArgs& a, int x0, int y0, int tx, int ty, double* tc) {

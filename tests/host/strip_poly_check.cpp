@@ -13,6 +13,10 @@
 //   bins     the same of the bins, of REF and DF, at any carrier down to none:
 //            within FP32 rounding (at their distance from the centre's) of the
 //            exact ones and inside the positions.
+//   split    whether a strip's pulses are shared out over waves: where its columns
+//            lie across range on images too small to fill the chip, not where
+//            each wave would stage a tile's positions; without the positions the
+//            kernels decide alike.
 //   root     the FP64 square root of the per-pixel fallback: two roundings.
 // Exit status 0 when the named check passes.
 #include <algorithm>
@@ -454,6 +458,44 @@ void check_root() {
   std::printf("largest error 2^%.2f\n", std::log2(worst));
 }
 
+void check_split() {
+  const int sizes[] = {128, 256, 512, 768, 1024, 1536};
+  for (int interp : {SARBP_INTERP_LINEAR, SARBP_INTERP_SINC8})
+    for (double spacing : {0.25, 0.5, 1.0})
+      for (int n : sizes)
+        for (int along = 0; along < 2; ++along) {
+          sarbp_grid g{};
+          g.ux[along] = spacing;
+          g.uy[1 - along] = spacing;
+          g.nx = g.ny = n;
+          g.origin[0] = g.origin[1] = -0.5 * n * spacing;
+          sarbp_params p{};
+          p.c = 299792458.0, p.fc = 9.6e9, p.dr = 0.1875, p.r0 = 4000, p.kaiser_beta = 6;
+          p.n_pulses = 512, p.n_samples = 8192, p.interp = interp;
+          std::vector<double> pos(3 * 512);
+          for (int m = 0; m < 512; ++m) pos[3 * m] = (m - 256) * 0.15, pos[3 * m + 1] = -4000, pos[3 * m + 2] = 3000;
+          for (int planned = 0; planned < 2; ++planned) {
+            const double* h = planned ? pos.data() : nullptr;
+            const sarbp_tuning t{4, 1, 4};
+            BpArgs a;
+            CHECK(plan_args(h, &g, &p, t, kRef, &a, nullptr) == SARBP_OK, "refused: %s", last_detail());
+            bool split = a.parts > 1;
+            if (split && a.split_limit > 0) split = split_wins(a, pos.data(), 4, a.split_limit);
+            CHECK(!planned || a.split_limit == 0, "planned with positions, left to the kernels");
+            CHECK(a.parts == 1 ? a.sum_pulses == INT32_MAX : (long)a.parts * a.sum_pulses >= 512, "%d sums of %d", a.parts,
+                  a.sum_pulses);
+            const bool sinc = interp == SARBP_INTERP_SINC8;
+            // measured: 256^2 always gains, 768^2 across range; along it sinc8
+            // loses from 768^2 on, linear from 1024^2; 1536^2 fills the chip
+            if (n <= 256 || (!along && n <= 768))
+              CHECK(split, "interp %d %g m %d^2 along %d planned %d: not split", interp, spacing, n, along, planned);
+            if (n >= 1536 || (along && n >= (sinc ? 768 : 1024)))
+              CHECK(!split, "interp %d %g m %d^2 along %d planned %d: split", interp, spacing, n, along, planned);
+            ++g_strips;
+          }
+        }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -464,6 +506,7 @@ int main(int argc, char** argv) {
   else if (!std::strcmp(name, "df_phase")) check_df_phase();
   else if (!std::strcmp(name, "bins")) check_bins();
   else if (!std::strcmp(name, "root")) check_root();
+  else if (!std::strcmp(name, "split")) check_split();
   else return std::fprintf(stderr, "unknown check %s\n", name), 2;
   std::printf("%s: %ld strips, %ld bounded, %d failures\n", name, g_strips, g_bounded, g_failures);
   return g_failures != 0;
