@@ -297,7 +297,8 @@ sarbp_status sarbp_get_tuning(sarbp_context* ctx, int32_t interp,
  * position-free defaults, or what sarbp_autotune without h_pos stored; an
  * all-class sarbp_set_tuning applies to both.  A call that takes a built-in
  * default of one column and 4 rows per lane for linear or sinc8 REF imaging
- * runs 8 rows on an image of 5120 or more 64 x 32 tiles. */
+ * runs 8 rows on an image of many 64 x 32 tiles: 5120 or more, linear 2048 or
+ * more below class 4. */
 sarbp_status sarbp_set_class_tuning(sarbp_context* ctx, int32_t interp,
                                     int32_t precision, int32_t dtype,
                                     int32_t size_class, const sarbp_tuning* tuning);

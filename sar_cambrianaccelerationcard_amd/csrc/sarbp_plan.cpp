@@ -220,32 +220,6 @@ sarbp_tuning default_tuning(int interp, int cls, int precision, bool positions) 
   return t;
 }
 
-// The built-in default for one job: on an image of many tiles the continuous
-// interpolators of SARBP_PREC_REF run 64 x 32 instead of 64 x 16 tiles, whose
-// row polynomials and FP64 setup serve twice the pixels.  Below about five
-// rounds of the 1024 workgroups that the chip holds, the coarser work items'
-// last round costs more than that: 1024 pulses over 3584^2 pixels (6272 tiles)
-// ran 4-11% faster at every spacing from 0.25 to 1 m, 2560^2 (3200 tiles)
-// between 2% faster and 5% slower, 1536^2 (1152 tiles) 5-40% slower.  Without
-// positions the widest windows' 64 x 32 tiles have LDS for fewer workgroups
-// per CU, which shows where there are few tiles: 512 pulses over 1024^2 pixels
-// took 814 / 809 / 1161 / 1229 us by 64 x 32 at 0.7 / 0.8 / 1 / 1.3 m, 672 /
-// 697 / 749 / 1288 by 64 x 16; over 2048^2 2362 / 2592 / 3633 / 4484 against
-// 2464 / 2577 / 3026 / 4405, over 3584^2 64 x 32 wins by 6-18%.
-sarbp_tuning job_tuning(int interp, int cls, int precision, bool positions, const sarbp_grid* g) {
-  sarbp_tuning t = default_tuning(interp, cls, precision, positions);
-  constexpr int64_t kManyTiles = 5 * 1024;
-  const int64_t tiles = (int64_t)((g->nx + 63) / 64) * ((g->ny + 31) / 32);
-  if (precision == SARBP_PREC_REF && interp != SARBP_INTERP_NEAREST && t.cols_per_lane == 1 && t.rows_per_lane == 4 &&
-      tiles >= kManyTiles)
-    t.rows_per_lane = 8;
-  constexpr int64_t kFewTiles = 1536;
-  if (precision == SARBP_PREC_REF && interp == SARBP_INTERP_SINC8 && !positions && cls == SARBP_SIZE_CLASSES - 1 &&
-      tiles <= kFewTiles)
-    t.rows_per_lane = 4;
-  return t;
-}
-
 // Largest |pixel - tile reference| the FP32 differential supports.  Two FP32
 // roundings grow with it: pp = |d|^2 - s^2 carries ~ulp(|d|^2) into
 // q = pp / (2R), a phase error ~ k ulp(|d|^2) / (2R) (at 48 m and R = 5 km,
@@ -308,6 +282,36 @@ double tile_radius(const sarbp_grid* g, int px, int py) {
     r = std::max(r, norm3(d));
   }
   return r;
+}
+
+// The built-in default for one job: on an image of many tiles the continuous
+// interpolators of SARBP_PREC_REF run 64 x 32 instead of 64 x 16 tiles, whose
+// row polynomials and FP64 setup serve twice the pixels.  Below about five
+// rounds of the 1024 workgroups that the chip holds, the coarser work items'
+// last round costs sinc8 more than that where columns lie across range: 1024
+// pulses over 3584^2 pixels (6272 tiles) ran 4-11% faster at every spacing from
+// 0.25 to 1 m, 2560^2 (3200 tiles) between 2% faster and 5% slower, 1536^2 (1152
+// tiles) 5-40% slower.  Linear gains from two rounds on, up to the windows of
+// 1 m pixels along range: 2048^2 of 0.25 m 567 -> 519 us across range, 687 -> 577
+// along it (256 pulses), 0.5 m 584 -> 551 and 762 -> 614; beyond the REF radius it
+// keeps 64 x 16 (1.6 m, 3584^2: 3017-3291 against 3458-3950).
+// Without positions a 64 x 32 tile of the widest windows has LDS for few pulses,
+// so images of up to one and a half tiles per CU take 64 x 16, which fit the CUs
+// in one round: 1024 x 768 of 1 m, across, along and at 45 degrees to range, 283 /
+// 553 / 557 us against 354 / 640 / 709 (256 pulses).  Larger ones gain across
+// range at 1 m (1280^2 577 against 914) but lose along it (1297 against 1113) and
+// at 1.3 m and beyond (1024^2 647 / 1326 / 1168 against 548 / 943 / 805).
+sarbp_tuning job_tuning(int interp, int cls, int precision, bool positions, const sarbp_grid* g) {
+  sarbp_tuning t = default_tuning(interp, cls, precision, positions);
+  if (precision != SARBP_PREC_REF || interp == SARBP_INTERP_NEAREST) return t;
+  constexpr int64_t kManyTiles = 5 * 1024, kManyLinear = 2 * 1024, kFewTiles = 384;
+  const int64_t tiles = (int64_t)((g->nx + 63) / 64) * ((g->ny + 31) / 32);
+  const bool linear = interp == SARBP_INTERP_LINEAR, near = tile_radius(g, 1, 8) <= kMaxTileRadius;
+  if (t.cols_per_lane == 1 && t.rows_per_lane == 4 &&
+      (linear ? near && tiles >= (cls < SARBP_SIZE_CLASSES - 1 ? kManyLinear : kManyTiles) : tiles >= kManyTiles))
+    t.rows_per_lane = 8;
+  if (!linear && !positions && cls == SARBP_SIZE_CLASSES - 1 && tiles <= kFewTiles) t.rows_per_lane = 4;
+  return t;
 }
 
 int plan_window(const sarbp_grid* g, const sarbp_params* p, int px, int py, const double* h_pos,
