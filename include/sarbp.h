@@ -323,8 +323,10 @@ typedef struct sarbp_autotune_result {
  * tiles to fill the device -- with HIP events on `stream`, and stores the
  * fastest as this context's tuning for the job's (interp, precision, dtype).
  * d_scratch receives the crop images and must hold scratch_pixels >=
- * crop_nx * crop_ny complex64 values.  The built-in default of the job's
- * size class stays unless a candidate is more than 2% faster.  The result is
+ * crop_nx * crop_ny complex64 values.  The built-in default of the job, timed
+ * as an untuned call launches it, stays unless a candidate is more than 2%
+ * faster; then `best` names it and the class's calls go on as untuned ones.  The
+ * result is
  * stored for the job's size class (sarbp_size_class) only, for calls with
  * host positions if h_pos is given, else for calls without (see
  * sarbp_set_class_tuning).  Synchronous.

@@ -91,14 +91,14 @@ namespace sarbp {
 
 // The context's tuning of a class, else its all-classes tuning, else the
 // built-in default (`positions`: for a plan that knows the antenna positions;
-// `g`: the job's grid, NULL for the class alone), and whether it is that.
+// `g`: the job's grid, NULL for the class alone), and whether it is that.  An
+// entry of no rows stands for the built-in default (sarbp_autotune).
 sarbp_tuning get_tuning(sarbp_context* ctx, int interp, int prec, int dtype, int cls, bool positions = true,
                         const sarbp_grid* g = nullptr, bool* builtin = nullptr) {
   if (builtin) *builtin = false;
   auto it = ctx->tuning.find(tuning_key(interp, prec, dtype, cls, positions));
-  if (it != ctx->tuning.end()) return it->second;
-  it = ctx->tuning.find(tuning_key(interp, prec, dtype, kAllClasses));
-  if (it != ctx->tuning.end()) return it->second;
+  if (it == ctx->tuning.end()) it = ctx->tuning.find(tuning_key(interp, prec, dtype, kAllClasses));
+  if (it != ctx->tuning.end() && it->second.rows_per_lane > 0) return it->second;
   if (builtin) *builtin = true;
   return g ? job_tuning(interp, cls, prec, positions, g) : default_tuning(interp, cls, prec, positions);
 }
@@ -569,9 +569,9 @@ sarbp_status sarbp_autotune(sarbp_context* ctx, const void* d_profiles, const do
     if (e0) (void)hipEventDestroy(e0);
     return hip_fail(e, "hipEventCreate");
   }
-  auto time_one = [&](const sarbp_tuning& t, double* ms, int* eff_p) -> sarbp_status {
+  auto time_one = [&](const sarbp_tuning& t, int prec, double* ms, int* eff_p) -> sarbp_status {
     BpArgs a;
-    sarbp_status r = plan_args(h_pos, &crop, &p, t, p.precision, &a, nullptr);
+    sarbp_status r = plan_args(h_pos, &crop, &p, t, prec, &a, nullptr);
     if (r != SARBP_OK) return r;
     *eff_p = a.pulses_per_stage;
     a.prof = d_profiles;
@@ -590,19 +590,22 @@ sarbp_status sarbp_autotune(sarbp_context* ctx, const void* d_profiles, const do
     *ms = f / reps;
     return SARBP_OK;
   };
-  // default first (built-in, ignoring any stored tuning)
+  // default first (built-in, ignoring any stored tuning), as an untuned call
+  // of the job launches it
   const int cls = size_class(grid, params, h_pos);
-  const sarbp_tuning def = job_tuning(p.interp, cls, p.precision, h_pos != nullptr, grid);
+  const Fitted def_fit =
+      fit_tuning(job_tuning(p.interp, cls, p.precision, h_pos != nullptr, grid), p.precision, grid, &p, h_pos, true);
+  const sarbp_tuning def = def_fit.t;
   int eff = 0;
   double def_ms = INFINITY;
-  st = time_one(def, &def_ms, &eff);
-  if (st == SARBP_ERR_UNSUPPORTED) st = SARBP_OK;  // default shape too large for this grid
+  st = time_one(def_fit.launch, def_fit.prec, &def_ms, &eff);
+  if (st == SARBP_ERR_UNSUPPORTED) st = SARBP_OK;
   sarbp_tuning best = def;
   best.pulses_per_stage = eff;
   double best_ms = def_ms;
   int n = std::isfinite(def_ms) ? 1 : 0;
   std::vector<std::tuple<int, int, int>> seen;
-  seen.emplace_back(def.cols_per_lane, def.rows_per_lane, eff);
+  seen.emplace_back(def_fit.launch.cols_per_lane, def_fit.launch.rows_per_lane, eff);
   const int shapes[][2] = {{1, 2}, {1, 4}, {1, 8}, {2, 2}, {2, 4}, {2, 8}, {4, 2}, {4, 4}};
   const int stages[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
   for (const auto& sh : shapes) {
@@ -622,7 +625,7 @@ sarbp_status sarbp_autotune(sarbp_context* ctx, const void* d_profiles, const do
       if (std::find(seen.begin(), seen.end(), key) != seen.end()) continue;
       seen.push_back(key);
       double ms = 0.0;
-      if ((st = time_one(t, &ms, &eff)) != SARBP_OK) break;
+      if ((st = time_one(t, p.precision, &ms, &eff)) != SARBP_OK) break;
       ++n;
       // a candidate replaces the built-in default only when it is more than
       // 2% faster: near-ties on one crop do not carry to the other jobs of
@@ -638,7 +641,10 @@ sarbp_status sarbp_autotune(sarbp_context* ctx, const void* d_profiles, const do
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   if (st != SARBP_OK) return st;
-  ctx->tuning[tuning_key(p.interp, p.precision, p.dtype, cls, h_pos != nullptr)] = best;
+  // the default is kept as such: what it is made to on other images of the
+  // class (job_tuning, cut strips) stays with it
+  ctx->tuning[tuning_key(p.interp, p.precision, p.dtype, cls, h_pos != nullptr)] =
+      best_ms < def_ms ? best : sarbp_tuning{0, 0, 0};
   out->best = best;
   out->best_ms = best_ms;
   out->default_ms = def_ms;

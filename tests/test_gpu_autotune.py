@@ -1,0 +1,60 @@
+"""The project autotuner's treatment of the built-in default."""
+import numpy as np
+import pytest
+
+from sar_cambrianaccelerationcard_amd import native
+
+pytestmark = pytest.mark.gpu
+
+KEY = (native.INTERP_SINC8, native.PREC_REF, native.DTYPE_C64)
+C0, DR = 299792458.0, 0.1875
+
+
+def _job(n, spacing, pulses, samples=4096, along=False):
+    pos = np.zeros((pulses, 3))
+    pos[:, 0], pos[:, 1], pos[:, 2] = np.linspace(-20, 20, pulses), -4000.0, 3000.0
+    u, v = ([0, spacing, 0], [spacing, 0, 0]) if along else ([spacing, 0, 0], [0, spacing, 0])
+    grid = native.make_grid([-0.5 * n * spacing, -0.5 * n * spacing, 0], u, v, n, n)
+    params = native.make_params(c=C0, fc=9.6e9, r0=5000.0 - 0.5 * samples * DR, dr=DR, n_pulses=pulses,
+                                n_samples=samples, interp="sinc8", precision="ref", dtype="c64", kaiser_beta=6.0)
+    return pos, grid, params
+
+
+def _tune(ctx, pos, grid, params, prof, d_pos, n):
+    import torch
+    scratch = torch.empty(n * n, dtype=torch.complex64, device="cuda")
+    return ctx.autotune(prof.data_ptr(), d_pos.data_ptr(), pos, grid, params, scratch.data_ptr(), n * n, 256,
+                        torch.cuda.current_stream().cuda_stream)
+
+
+def test_a_kept_default_stays_the_default():
+    """Pixels too coarse for every REF shape: no candidate can win, and calls of
+    the class go on as untuned ones, a small image's cut strips included (bit
+    for bit), whatever all-class tuning was set before."""
+    import torch
+    pulses = 48
+    # (columns along range give the chip the coarse image's class)
+    coarse, chip = _job(256, 1.6, pulses), _job(96, 1.2, pulses, along=True)
+    prof = torch.randn((pulses, 4096, 2), device="cuda")
+    d_pos = torch.from_numpy(coarse[0]).cuda()
+    cls = native.size_class(coarse[1], coarse[2], coarse[0])
+
+    def image(ctx, pos, grid, params):
+        img = torch.zeros((96, 96), dtype=torch.complex64, device="cuda")
+        ctx.plan(pos, grid, params).execute(prof.data_ptr(), d_pos.data_ptr(), img.data_ptr(),
+                                            torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        return img.cpu().numpy().view(np.uint64)
+
+    fresh, tuned = native.Context(0), native.Context(0)
+    try:
+        assert native.size_class(chip[1], chip[2], chip[0]) == cls
+        tuned.set_tuning(*KEY, 8, 1, 2)
+        r = _tune(tuned, *coarse, prof, d_pos, 256)
+        print(f"  {r}", flush=True)
+        assert r["n_candidates"] == 1 and r["best_ms"] == r["default_ms"] < 1e9
+        assert tuned.get_class_tuning(*KEY, cls) == fresh.get_class_tuning(*KEY, cls)
+        assert np.array_equal(image(tuned, *chip), image(fresh, *chip))
+    finally:
+        fresh.close()
+        tuned.close()
