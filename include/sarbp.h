@@ -320,7 +320,8 @@ typedef struct sarbp_autotune_result {
  * configuration whose LDS footprint fits, on a centred crop of the given job
  * (all pulses, the plan the optional host positions allow) that keeps up to
  * max(max_crop_px, 4096) columns and holds about max_crop_px^2 pixels -- enough
- * tiles to fill the device -- with HIP events on `stream`, and stores the
+ * tiles to fill the device -- in the form that the whole image's launch takes,
+ * with HIP events on `stream`, and stores the
  * fastest as this context's tuning for the job's (interp, precision, dtype).
  * d_scratch receives the crop images and must hold scratch_pixels >=
  * crop_nx * crop_ny complex64 values.  The built-in default of the job, timed

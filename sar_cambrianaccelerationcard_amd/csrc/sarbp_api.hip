@@ -569,9 +569,25 @@ sarbp_status sarbp_autotune(sarbp_context* ctx, const void* d_profiles, const do
     if (e0) (void)hipEventDestroy(e0);
     return hip_fail(e, "hipEventCreate");
   }
+  // The whole image's launch on the crop: its windows, its LDS and whether its
+  // pulses are shared out over waves, which the crop's own size would decide
+  // otherwise (a 4096 x 256 crop of 4096^2 pixels has few enough strips to share
+  // them, the image has not).
+  auto plan_crop = [&](const sarbp_tuning& t, int prec, BpArgs* a) -> sarbp_status {
+    BpArgs c;
+    sarbp_status r = plan_args(h_pos, grid, &p, t, prec, a, nullptr);
+    if (r == SARBP_OK) r = plan_args(h_pos, &crop, &p, t, prec, &c, nullptr);
+    if (r != SARBP_OK) return r;
+    std::memcpy(a->origin, c.origin, sizeof a->origin);
+    a->nx = c.nx;
+    a->ny = c.ny;
+    a->tiles_x = c.tiles_x;
+    a->tiles_y = c.tiles_y;
+    return SARBP_OK;
+  };
   auto time_one = [&](const sarbp_tuning& t, int prec, double* ms, int* eff_p) -> sarbp_status {
     BpArgs a;
-    sarbp_status r = plan_args(h_pos, &crop, &p, t, prec, &a, nullptr);
+    sarbp_status r = plan_crop(t, prec, &a);
     if (r != SARBP_OK) return r;
     *eff_p = a.pulses_per_stage;
     a.prof = d_profiles;
@@ -605,7 +621,11 @@ sarbp_status sarbp_autotune(sarbp_context* ctx, const void* d_profiles, const do
   double best_ms = def_ms;
   int n = std::isfinite(def_ms) ? 1 : 0;
   std::vector<std::tuple<int, int, int>> seen;
-  seen.emplace_back(def_fit.launch.cols_per_lane, def_fit.launch.rows_per_lane, eff);
+  {
+    BpArgs d;
+    const bool shared = plan_crop(def_fit.launch, def_fit.prec, &d) == SARBP_OK && d.parts > 1 && !(d.split_limit > 0.0f);
+    seen.emplace_back(def_fit.launch.cols_per_lane, def_fit.launch.rows_per_lane, shared ? 0 : eff);
+  }
   const int shapes[][2] = {{1, 2}, {1, 4}, {1, 8}, {2, 2}, {2, 4}, {2, 8}, {4, 2}, {4, 4}};
   const int stages[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
   for (const auto& sh : shapes) {
@@ -617,11 +637,14 @@ sarbp_status sarbp_autotune(sarbp_context* ctx, const void* d_profiles, const do
       t.rows_per_lane = sh[1];
       t.pulses_per_stage = P;
       BpArgs probe;
-      if (plan_args(h_pos, &crop, &p, t, p.precision, &probe, nullptr) != SARBP_OK) continue;
+      if (plan_crop(t, p.precision, &probe) != SARBP_OK) continue;
+      // waves that share the pulses out have no stage to set the depth of
+      const bool shared = probe.parts > 1 && !(probe.split_limit > 0.0f);
+      if (shared) t.pulses_per_stage = def.pulses_per_stage;
       // fewer than 4 pulses per stage only pay where 4 would leave fewer
       // than 4 workgroups per CU (40 KiB of LDS each)
-      if (P < 4 && lds_layout(probe.kernel_interp, probe.win, 4).total <= 40 * 1024) continue;
-      const auto key = std::make_tuple(sh[0], sh[1], probe.pulses_per_stage);
+      if (!shared && P < 4 && lds_layout(probe.kernel_interp, probe.win, 4).total <= 40 * 1024) continue;
+      const auto key = std::make_tuple(sh[0], sh[1], shared ? 0 : probe.pulses_per_stage);
       if (std::find(seen.begin(), seen.end(), key) != seen.end()) continue;
       seen.push_back(key);
       double ms = 0.0;

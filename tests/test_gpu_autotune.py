@@ -58,3 +58,31 @@ def test_a_kept_default_stays_the_default():
     finally:
         fresh.close()
         tuned.close()
+
+
+def test_shared_pulses_are_one_candidate_a_shape():
+    """A small image's one-column launches share its pulses out over waves, which
+    no stage depth changes: one candidate per row count, and every planned depth
+    of the other shapes."""
+    import torch
+    n, pulses = 128, 64
+    pos, grid, params = _job(n, 0.25, pulses)
+    prof = torch.randn((pulses, 4096, 2), device="cuda")
+    d_pos = torch.from_numpy(pos).cuda()
+    ctx = native.Context(0)
+    try:
+        depths = set()
+        for cols, rows in ((2, 2), (2, 4), (2, 8), (4, 2), (4, 4)):
+            for P in (1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64):
+                ctx.set_tuning(*KEY, rows, cols, P)
+                i = ctx.plan(pos, grid, params).info()
+                assert (i["cols_per_lane"], i["rows_per_lane"]) == (cols, rows)
+                if i["pulses_per_stage"] >= 4:
+                    depths.add((cols, rows, i["pulses_per_stage"]))
+        ctx.set_tuning(*KEY, 0, 0, 0)
+        r = _tune(ctx, pos, grid, params, prof, d_pos, n)
+        print(f"  {r}, depths of the wider shapes {len(depths)}", flush=True)
+        # the default is one of the three row counts
+        assert r["n_candidates"] == 3 + len(depths)
+    finally:
+        ctx.close()
