@@ -321,7 +321,8 @@ typedef struct sarbp_autotune_result {
  * (all pulses, the plan the optional host positions allow) that keeps up to
  * max(max_crop_px, 4096) columns and holds about max_crop_px^2 pixels -- enough
  * tiles to fill the device -- in the form that the whole image's launch takes,
- * with HIP events on `stream`, and stores the
+ * tiles of another size than the default's only where the crop is the image or
+ * holds four rounds of them, with HIP events on `stream`, and stores the
  * fastest as this context's tuning for the job's (interp, precision, dtype).
  * d_scratch receives the crop images and must hold scratch_pixels >=
  * crop_nx * crop_ny complex64 values.  The built-in default of the job, timed

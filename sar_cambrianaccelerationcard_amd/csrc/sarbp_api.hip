@@ -628,9 +628,19 @@ sarbp_status sarbp_autotune(sarbp_context* ctx, const void* d_profiles, const do
   }
   const int shapes[][2] = {{1, 2}, {1, 4}, {1, 8}, {2, 2}, {2, 4}, {2, 8}, {4, 2}, {4, 4}};
   const int stages[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
+  // Part of an image ranks tiles of other sizes by their last round: 4096 x 256
+  // pixels of 4096^2, half a round of 64 x 32 tiles, took 64 x 16 for faster,
+  // which are 14-20% slower on the whole.  Those are compared where the crop
+  // holds four rounds of the larger tile (or all of the image).
+  const int def_px = def_fit.launch.cols_per_lane * def_fit.launch.rows_per_lane;
+  auto crop_ranks = [&](int tile_px) {
+    const int64_t px = (int64_t)crop.nx * crop.ny;
+    return tile_px == def_px || (crop.nx == grid->nx && crop.ny == grid->ny) ||
+           px >= (int64_t)4 * 4 * ctx->n_cu * kThreads * std::max(tile_px, def_px);
+  };
   for (const auto& sh : shapes) {
     if (st != SARBP_OK) break;
-    if (!tile_shape_supported(p.precision, sh[0], sh[1])) continue;
+    if (!tile_shape_supported(p.precision, sh[0], sh[1]) || !crop_ranks(sh[0] * sh[1])) continue;
     for (int P : stages) {
       sarbp_tuning t;
       t.cols_per_lane = sh[0];

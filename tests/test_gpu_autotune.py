@@ -20,10 +20,10 @@ def _job(n, spacing, pulses, samples=4096, along=False):
     return pos, grid, params
 
 
-def _tune(ctx, pos, grid, params, prof, d_pos, n):
+def _tune(ctx, pos, grid, params, prof, d_pos, n, crop_px=256):
     import torch
     scratch = torch.empty(n * n, dtype=torch.complex64, device="cuda")
-    return ctx.autotune(prof.data_ptr(), d_pos.data_ptr(), pos, grid, params, scratch.data_ptr(), n * n, 256,
+    return ctx.autotune(prof.data_ptr(), d_pos.data_ptr(), pos, grid, params, scratch.data_ptr(), n * n, crop_px,
                         torch.cuda.current_stream().cuda_stream)
 
 
@@ -84,5 +84,32 @@ def test_shared_pulses_are_one_candidate_a_shape():
         print(f"  {r}, depths of the wider shapes {len(depths)}", flush=True)
         # the default is one of the three row counts
         assert r["n_candidates"] == 3 + len(depths)
+    finally:
+        ctx.close()
+
+
+def test_a_small_crop_ranks_tiles_of_the_defaults_size_only():
+    """512 x 8 pixels of 512 x 512: tiles of other sizes would be ranked by their
+    last round, so only the default's (4 pixels per lane) are timed."""
+    import torch
+    n, pulses = 512, 64
+    pos, grid, params = _job(n, 0.25, pulses)
+    prof = torch.randn((pulses, 4096, 2), device="cuda")
+    d_pos = torch.from_numpy(pos).cuda()
+    ctx = native.Context(0)
+    try:
+        depths = set()
+        for P in (1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64):
+            ctx.set_tuning(*KEY, 2, 2, P)
+            i = ctx.plan(pos, grid, params).info()
+            assert (i["cols_per_lane"], i["rows_per_lane"]) == (2, 2)
+            if i["pulses_per_stage"] >= 4:
+                depths.add(i["pulses_per_stage"])
+        ctx.set_tuning(*KEY, 0, 0, 0)
+        r = _tune(ctx, pos, grid, params, prof, d_pos, n, 64)
+        print(f"  {r}, depths of 2 x 2 {len(depths)}", flush=True)
+        assert r["crop"] == [512, 8]
+        assert r["cols_per_lane"] * r["rows_per_lane"] == 4
+        assert r["n_candidates"] == 1 + len(depths)
     finally:
         ctx.close()
