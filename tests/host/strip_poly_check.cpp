@@ -17,6 +17,9 @@
 //            lie across range on images too small to fill the chip, not where
 //            each wave would stage a tile's positions; without the positions the
 //            kernels decide alike.
+//   launch   random planned launches, plain and batched: their LDS within the
+//            budget, room for a whole window in it, every pulse in a partial sum,
+//            the same sums in both.
 //   root     the FP64 square root of the per-pixel fallback: two roundings.
 // Exit status 0 when the named check passes.
 #include <algorithm>
@@ -496,6 +499,67 @@ void check_split() {
         }
 }
 
+void check_launch() {
+  // registers allow 4 workgroups per CU; LDS in 512-B blocks
+  set_occupancy_source([](int, int, int, int, int, size_t shm) {
+    return std::max(1, std::min(4, (int)(160 * 1024 / 512 / ((shm + 16 + 511) / 512))));
+  });
+  Rng rng(23);
+  long cut = 0, shared = 0, chosen = 0;
+  for (int i = 0; i < 20000; ++i) {
+    sarbp_grid g{};
+    const double sx = log_uniform(rng, 0.02, 8.0), sy = sx * log_uniform(rng, 0.2, 5.0), ang = uniform(rng, 0, 6.2831853);
+    g.ux[0] = sx * std::cos(ang), g.ux[1] = sx * std::sin(ang);
+    g.uy[0] = -sy * std::sin(ang), g.uy[1] = sy * std::cos(ang);
+    g.nx = (int)log_uniform(rng, 1, 9000);
+    g.ny = (int)log_uniform(rng, 1, 9000);
+    sarbp_params p{};
+    p.c = 299792458.0, p.fc = 9.6e9, p.dr = log_uniform(rng, 0.05, 2.0), p.kaiser_beta = 6;
+    p.n_pulses = rng() % 20 ? 1 + (int)(rng() % 300) : (int)(rng() % 2);
+    p.n_samples = 4096;
+    p.interp = 1 + (int)(rng() % 2);
+    p.precision = rng() % 4 ? SARBP_PREC_REF : SARBP_PREC_DF;
+    const double R = log_uniform(rng, 300, 1e6);
+    std::vector<double> pos(3 * (size_t)p.n_pulses + 3);
+    for (int m = 0; m < p.n_pulses; ++m) pos[3 * m] = m * 0.2, pos[3 * m + 1] = -0.8 * R, pos[3 * m + 2] = 0.6 * R;
+    const double* h = rng() % 2 ? pos.data() : nullptr;
+    const int cls = size_class(&g, &p, h);
+    sarbp_tuning t = job_tuning(p.interp, cls, p.precision, h != nullptr, &g);
+    const bool builtin = rng() % 2;
+    if (!builtin) {
+      static const int shapes[][2] = {{1, 2}, {1, 4}, {1, 8}, {2, 2}, {2, 4}, {2, 8}, {4, 2}, {4, 4}};
+      const int* sh = shapes[rng() % 8];
+      t = sarbp_tuning{sh[1], sh[0], 1 + (int)(rng() % 256)};
+      if (check_tuning(p.precision, &t) != SARBP_OK) continue;
+    }
+    const Fitted f = fit_tuning(t, p.precision, &g, &p, h, builtin);
+    BpArgs a, b, whole;
+    const sarbp_status st = plan_args(h, &g, &p, f.launch, f.prec, &a, nullptr);
+    // a cut tile is refused only where the tuned one is
+    CHECK((plan_args(h, &g, &p, f.t, f.prec, &whole, nullptr) == SARBP_OK) == (st == SARBP_OK), "cut tile refused: %s", last_detail());
+    if (st != SARBP_OK) continue;
+    ++g_strips;
+    CHECK(plan_args(h, &g, &p, f.launch, f.prec, &b, nullptr, true) == SARBP_OK, "batched plan refused");
+    for (const BpArgs* x : {&a, &b}) {
+      const int room = window_room(x->kernel_interp, x->win);
+      CHECK(x->pool >= room, "%d staged positions, a window has %d", x->pool, room);
+      CHECK(launch_lds(*x) <= kLdsBudget, "%zu bytes of LDS", launch_lds(*x));
+      CHECK(x->parts >= 1 && x->parts <= kMaxParts && x->sum_pulses >= 1, "%d parts of %d", x->parts, x->sum_pulses);
+      CHECK(x->parts == 1 ? x->sum_pulses >= p.n_pulses : (long)x->parts * x->sum_pulses >= p.n_pulses, "%d parts of %d, %d pulses",
+            x->parts, x->sum_pulses, p.n_pulses);
+      CHECK(x->parts == 1 || f.launch.cols_per_lane == 1, "parts of %d columns", f.launch.cols_per_lane);
+      CHECK(x->split_limit == 0 || (x->parts > 1 && !h), "limit %g, %d parts", x->split_limit, x->parts);
+    }
+    CHECK(a.parts == b.parts && a.sum_pulses == b.sum_pulses && a.split_limit == b.split_limit && a.win == b.win &&
+              a.kernel_interp == b.kernel_interp, "plain and batched plans differ");
+    cut += f.launch.rows_per_lane != f.t.rows_per_lane;
+    shared += a.parts > 1;
+    chosen += a.split_limit > 0;
+  }
+  CHECK(cut > 100 && shared > 100 && chosen > 100, "%ld cut, %ld shared, %ld left to the kernels", cut, shared, chosen);
+  set_occupancy_source(nullptr);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -507,6 +571,7 @@ int main(int argc, char** argv) {
   else if (!std::strcmp(name, "bins")) check_bins();
   else if (!std::strcmp(name, "root")) check_root();
   else if (!std::strcmp(name, "split")) check_split();
+  else if (!std::strcmp(name, "launch")) check_launch();
   else return std::fprintf(stderr, "unknown check %s\n", name), 2;
   std::printf("%s: %ld strips, %ld bounded, %d failures\n", name, g_strips, g_bounded, g_failures);
   return g_failures != 0;

@@ -23,7 +23,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["window", "ref", "df", "df_phase", "bins", "root", "split"])
+@pytest.mark.parametrize("check", ["window", "ref", "df", "df_phase", "bins", "root", "split", "launch"])
 def test_strip_polynomials(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=300)
     print(r.stdout, r.stderr[-4000:])
