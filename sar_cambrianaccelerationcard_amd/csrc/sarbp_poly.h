@@ -395,6 +395,7 @@ SARBP_HD RowTerms comp_row(const float4& p0, const float4& p1, const float4& p2,
 // against split 768^2 and 1024^2 ones, columns across, along and at 45 degrees
 // to range at 0.25 to 1.6 m: within 25% of the measured ratios of 0.9 to 3.3.
 SARBP_HD float split_cost(int interp, int prec, int rows, float strip, float tile) {
+#pragma clang fp contract(off)
   const bool sinc = sinc_rows(interp) > 0;
   const float pixels = (sinc ? 6.25f : 37.0f) * (float)rows;
   const float pieces = ceilf(strip / (float)(kSplitStage / room_bytes(interp)));
@@ -404,13 +405,17 @@ SARBP_HD float split_cost(int interp, int prec, int rows, float strip, float til
 // Positions that a strip of 64 columns by `rows` rows touches, of range steps dx
 // and dy (m) a pixel.
 SARBP_HD float touched(double dx, double dy, int rows, double inv_dr) {
+#pragma clang fp contract(off)
   return (float)((dx * (kTileX - 1) + dy * (rows - 1)) * inv_dr) + 3.5f;
 }
 
 // Whether a job's strips cost less than `limit` split, by the mean range steps at
 // two quarter points of the image from the first, the middle and the last of
-// its antenna positions.  A position that is no number does not split.
+// its antenna positions.  A position that is no number does not split.  Two
+// launches of one call ask, and each images what the other leaves: they have to
+// round alike, so here as in the functions above the compiler contracts nothing.
 SARBP_HD bool split_wins(const BpArgs& a, const double* pos, int rows, float limit) {
+#pragma clang fp contract(off)
   double dx = 0.0, dy = 0.0;
   for (int m = 0; m < 6; ++m) {
     const double* p = pos + 3 * (size_t)(m % 3 == 0 ? 0 : (m % 3 == 1 ? a.n_pulses / 2 : a.n_pulses - 1));
