@@ -277,8 +277,9 @@ struct PolySetup {
   // Where the strip is not bounded: the planned window about the tile reference
   // pixel, every pixel's bin clamped into it.
   SARBP_HD void whole_window(const BpArgs& a, const double* tc, const double* pos) {
+#pragma clang fp contract(off)
     const double ex = tc[0] - pos[0], ey = tc[1] - pos[1], ez = tc[2] - pos[2];
-    const double bc = floor((sqrt(ex * ex + ey * ey + ez * ez) - a.r0) * a.inv_dr) - (double)a.half;
+    const double bc = floor((sqrt(fma(ez, ez, fma(ey, ey, ex * ex))) - a.r0) * a.inv_dr) - (double)a.half;
     first = (int)fmax(fmin(bc, 2.0e9), -2.0e9) + (sinc_rows(INTERP) > 0 ? 3 : 0);
     n = window_room(INTERP, a.win);
     mode = 2;
@@ -435,14 +436,21 @@ SARBP_HD bool split_wins(const BpArgs& a, const double* pos, int rows, float lim
                     touched(dx, dy, kWaves * rows, a.inv_dr)) < limit;
 }
 
+SARBP_HD double dot_fma(const double* u, const double* v) { return fma(u[2], v[2], fma(u[1], v[1], u[0] * v[0])); }
+
 // The setup's constants of one tile: its reference pixel and the grid steps'
-// products (kept in LDS, not in 12 registers through the pixel loop).
+// products (kept in LDS, not in 12 registers through the pixel loop).  Here, in
+// strip_centre and in whole_window the FMAs are written out: left to the
+// compiler, kernels that image the same job might round them differently.
 SARBP_HD void tile_constants(const BpArgs& a, int x0, int y0, int tx, int ty, double* tc) {
   const int ic = x0 + tx / 2, jc = y0 + ty / 2;
-  for (int k = 0; k < 3; ++k) tc[k] = a.origin[k] + ic * a.ux[k] + jc * a.uy[k];
-  tc[3] = a.ux[0] * a.ux[0] + a.ux[1] * a.ux[1] + a.ux[2] * a.ux[2];
-  tc[4] = a.ux[0] * a.uy[0] + a.ux[1] * a.uy[1] + a.ux[2] * a.uy[2];
-  tc[5] = a.uy[0] * a.uy[0] + a.uy[1] * a.uy[1] + a.uy[2] * a.uy[2];
+  for (int k = 0; k < 3; ++k) tc[k] = fma((double)jc, a.uy[k], fma((double)ic, a.ux[k], a.origin[k]));
+  tc[3] = dot_fma(a.ux, a.ux);
+  tc[4] = dot_fma(a.ux, a.uy);
+  tc[5] = dot_fma(a.uy, a.uy);
 }
+
+// A strip's centre, yc rows from the tile reference pixel.
+SARBP_HD double strip_centre(const BpArgs& a, const double* tc, double yc, int k) { return fma(yc, a.uy[k], tc[k]); }
 
 }  // namespace sarbp
