@@ -148,7 +148,11 @@ __device__ __forceinline__ void dit(const float2* x, int o, const float2* tw, fl
 // twiddles into the DFT's butterflies: 192 FMAs and 7 products, where twiddled
 // inputs ahead of a 4 x 4 DFT take 29 + 8 products and 144 sums.  4096 lines of
 // 3414 samples (chirp-z on 8192 points, there and back) ran 327 us, now 300
-// (12% fewer vector instructions in the kernel); error against FP64 unchanged.
+// (12% fewer vector instructions in the kernel).  Its twiddles are w^1, w^2, w^4
+// and w^8 of the table's w; with w^2 from the table too, and not squared from w,
+// the 3072 x 2048 scene's error against FP64 is 7.3e-7, 9.3e-7 without and
+// 9.2e-7 by twiddled inputs, in the same time (w^4 as well: a sixth less error,
+// 1.4% slower).
 // The smaller radices keep twiddled inputs: range compression stores these
 // sums as bf16 words, which stay bit for bit, and gained 3%.
 template <int LG, int R, bool INV>
@@ -167,7 +171,8 @@ __device__ __forceinline__ void twiddle_dft(float2* y, const float2* __restrict_
     constexpr float sg = INV ? 1.0f : -1.0f;
     const float2 w1 = w[1];
     w[8] = w1;
-    w[4] = cmul(w1, w1);
+    w[4] = tw[(2 * k) << (LG - lns - LGR)];
+    if (INV) w[4].y = -w[4].y;
     w[2] = cmul(w[4], w[4]);
     w[1] = cmul(w[2], w[2]);
     w[5] = cmul(w[4], make_float2(c2, sg * c2));

@@ -1,11 +1,14 @@
-"""FP32 rounding against the FP64 oracle: images no further from it than those of
-the kernels that the present ones took the place of (a range expansion per
-pixel), whose measured errors are the limits."""
+"""FP32 rounding against the FP64 oracles: images and omega-K scenes no further
+from them than the kernels that the present ones took the place of (a range
+expansion per pixel; twiddled inputs of a 4 x 4 DFT), whose measured errors are
+the limits."""
 import numpy as np
 import pytest
 
 import oracle as O
+import wk_oracle as W
 from sar_cambrianaccelerationcard_amd import native
+from sar_cambrianaccelerationcard_amd import omegak
 
 pytestmark = pytest.mark.gpu
 
@@ -50,4 +53,24 @@ def test_image_rounding(interp, nx, ny, pulses, spacing, limit):
         ctx.close()
     err = np.linalg.norm(img.cpu().numpy() - ref) / np.linalg.norm(ref)
     print(f"  {interp} {nx} x {ny} of {spacing} m, {pulses} pulses: rel_l2={err:.3e}", flush=True)
+    assert err <= limit
+
+
+@pytest.mark.parametrize("na_in,nr_in,range_ref,limit", [(3072, 2048, "r0", 9.22e-7),
+                                                            (701, 613, "centre", 8.45e-7)])
+def test_omega_k_rounding(na_in, nr_in, range_ref, limit):
+    from sar_cambrianaccelerationcard_amd import device
+    rng = np.random.default_rng(na_in)
+    echo = rng.standard_normal((na_in, nr_in, 2)).astype(np.float32).view(np.complex64)[..., 0]
+    wp = omegak.radarsat_scene(na_in=na_in, nr_in=nr_in).params(range_ref=range_ref)
+    ref = W.omega_k(echo, c=wp.c, f0=wp.f0, fs=wp.fs, prf=wp.prf, kr=wp.kr, vr=wp.vr, r0=wp.r0, f_nc=wp.f_nc,
+                    taps=wp.taps, window=wp.window, range_ref=wp.range_ref)
+    ctx = native.Context(0)
+    try:
+        import torch
+        got = device.omega_k(ctx, torch.from_numpy(np.ascontiguousarray(echo)).to("cuda:0"), wp).cpu().numpy()
+    finally:
+        ctx.close()
+    err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    print(f"  omega-K {na_in} x {nr_in} {range_ref}: rel_l2={err:.3e}", flush=True)
     assert err <= limit
