@@ -58,16 +58,18 @@ typedef enum sarbp_interp {
 } sarbp_interp;
 
 typedef enum sarbp_precision {
-  /* FP64 per-(tile, pulse) reference range and phase, FP32 per-pixel
-   * differential with exact modular phase reduction.  Default.  The FP32
-   * differential bounds a tile's radius (48 m at 5 km, more at longer
-   * range); a job whose grid no tile shape fits runs SARBP_PREC_DF. */
+  /* FP64 reference range and phase per pulse and strip of at most 1024
+   * pixels (nearest: and tile), FP32 differential with exact modular phase
+   * reduction: a polynomial over the strip (nearest, and strips too coarse or
+   * too near for one: pixel by pixel).  Default.  The FP32 differential bounds
+   * a tile's radius (48 m at 5 km, more at longer range); a job whose grid no
+   * tile shape fits runs SARBP_PREC_DF. */
   SARBP_PREC_REF = 0,
   SARBP_PREC_F64 = 1, /* FP64 slant range and phase for every pixel-pulse    */
   SARBP_PREC_F32 = 2, /* FP32 positions, range and phase (inaccurate)         */
-  /* FP64 per-(tile, pulse) reference plus a compensated double-float
-   * (FP32 pair) per-pixel differential range and phase: no tile-radius
-   * limit, about half the REF rate. */
+  /* As SARBP_PREC_REF to a higher order, its large phase terms unrounded
+   * (strips beyond that: FP64 per pixel; nearest: FP32 pairs per pixel): no
+   * tile-radius limit, about 0.85 of the REF rate. */
   SARBP_PREC_DF = 3
 } sarbp_precision;
 
@@ -190,10 +192,10 @@ sarbp_status sarbp_launch_generate_echo(sarbp_cf32* Srnm, const float* Ptarget,
 /*
  * A plan fixes the launch configuration for one geometry.  sarbp_backproject
  * plans from the grid alone (range window sized by the triangle inequality,
- * second-order range expansion); a plan made from the host copy of the
- * antenna positions bounds the line-of-sight directions and the minimum slant
- * range over the whole scene, which gives shorter LDS windows and, where the
- * bound allows it, the cheaper first-order range expansion.  The plan stays
+ * second-order range expansion for nearest); a plan made from the host copy of
+ * the antenna positions bounds the line-of-sight directions and the minimum
+ * slant range over the whole scene, which gives shorter LDS windows and, for
+ * nearest where the bound allows it, the cheaper first-order range expansion.  The plan stays
  * valid for any positions inside the bounds computed at creation (the device
  * positions passed to sarbp_plan_execute must be the ones planned for).
  */
@@ -205,10 +207,13 @@ typedef struct sarbp_plan_info {
   int32_t window;               /* LDS range window per pulse, samples       */
   int32_t pulses_per_stage;     /* pulses staged per barrier interval        */
   int32_t rows_per_lane, cols_per_lane;
-  int32_t range_order;          /* 1 if the first-order expansion holds over
-                                   the whole scene, else 0 (chosen per stage) */
+  int32_t range_order;          /* nearest: 1 if the first-order expansion
+                                   holds over the whole scene, else 0 (chosen
+                                   per pulse)                                */
   int32_t lds_bytes;            /* dynamic LDS per workgroup                 */
-  double max_phase_err_rad;     /* bound on the expansion truncation error   */
+  double max_phase_err_rad;     /* bound on the truncation error of nearest's
+                                   expansion (linear, sinc8: REF 5e-6 rad, DF
+                                   8e-6, by each strip's own test)           */
   int32_t sinc8_halves;         /* SINC8 kernel: 2 = half-bin degree-5 tap
                                    polynomials, 1 = whole-bin degree 7; 0 for
                                    other interpolators (chosen per launch)   */
@@ -241,8 +246,10 @@ const char* sarbp_last_error_detail(void);
  * more workgroup share a CU (a job's window sets the LDS per pulse), down to
  * 4 pulses for a plain launch (sarbp_plan_get_info reports the depth planned)
  * and to 1 for a job of a batch or a server.  Linear and sinc8 launches of
- * SARBP_PREC_REF take at most the LDS that lets 4 workgroups share a CU, and
- * pack it with as many pulses as fit at the length they touch.
+ * SARBP_PREC_REF and _DF take at most the LDS that lets 4 workgroups share a
+ * CU (fewer where the image has fewer tiles), and pack it with as many pulses
+ * as fit at the length they touch; images of few strips share their pulses out
+ * over waves instead, for which the depth means nothing.
  * The depth changes no bit of an image.  Where no tuning is set, linear and
  * sinc8 images of few 64 x 4 pixel strips (REF, DF; up to 32 rows_per_lane) are
  * launched with 2 rows per lane, or (8 rows, up to 640) with 4;

@@ -602,6 +602,8 @@ sarbp_status plan_args(const double* h_pos, const sarbp_grid* g,
   // occupancy and fit down to 1 pulse (64 mixed jobs: 191.7 ms that way,
   // 217.0 ms stopping at 4, same box).  The depth changes no result bit:
   // each pixel adds its pulses in pulse order whatever the stages.
+  // Row polynomials take this depth as a bound on their pool and setup batch,
+  // whatever their own LDS, which stage_pool fits.
   auto per_cu = [&](int q) {
     return kernel_occupancy(kinterp, kprec, p->dtype, px, py, lds_layout(kinterp, win, q).total);
   };

@@ -92,8 +92,8 @@ SARBP_HD constexpr double bin_scale() {
 // strip's positions keep them inside.
 // 4096 x 4096 x 4096 pulses, 0.25 m, sinc8: 59 ms with the expansion per pixel
 // (36.9 VALU instructions and 28.6 issue slots per pixel-pulse, 1 x 4 pixels
-// per lane), 48.3 ms this way at 1 x 8 (27 in the pixel loop), bound by the
-// VALU issue slots at 84% with the LDS pipe 65% busy beside them.
+// per lane), 49.5-50.3 ms this way at 1 x 8 (30.1 and 23.8), bound by the VALU
+// issue slots, 89% used, with the LDS pipe 66% busy beside them.
 constexpr float kPolyTol[2] = {1.5e-6f, 5e-6f};  // rad, modes 0 and 1
 // The bin has its own limit, which rules at low carriers and, against the
 // phase's y^3, for rows that are long against dr: its y^3 is the best fit in y.
